@@ -154,6 +154,23 @@ def test_route_permute_is_a_stable_sort(hip_ext, t, k, e):
     assert torch.equal(offsets.cpu(), torch.cat((torch.zeros(1, dtype=torch.int64), counts.cumsum(0))))
 
 
+# 3072 routes are the one-workgroup sort's last size; beyond, one workgroup per
+# 1024 routes (the last one partly filled), per 2048 above 65536
+@pytest.mark.parametrize("routes,e,hot", [(3073, 60, 0.0), (4096, 256, 0.0), (8191, 64, 0.9), (32760, 64, 0.0),
+                                          (65537, 128, 0.3)])
+def test_route_permute_many_routes(hip_ext, routes, e, hot):
+    note(f"permute routes={routes} e={e} hot={hot}")
+    g = torch.Generator().manual_seed(routes)
+    ids = torch.randint(-2, e + 2, (routes,), generator=g)  # some ids out of range
+    ids[torch.rand(routes, generator=g) < hot] = e // 2
+    order, offsets = hip_ext.route_permute(ids.view(-1, 1).to(DEV), e)
+    keep = ((ids >= 0) & (ids < e)).nonzero().flatten()
+    ref = keep[torch.argsort(ids[keep], stable=True)]
+    counts = torch.bincount(ids[keep], minlength=e)
+    assert torch.equal(offsets.cpu(), torch.cat((torch.zeros(1, dtype=torch.int64), counts.cumsum(0))))
+    assert torch.equal(order.cpu()[:keep.numel()], ref)
+
+
 def test_route_permute_drops_invalid_ids(hip_ext):
     note("permute invalid ids")
     idx = torch.tensor([[3, -1], [70, 3], [0, 5]])

@@ -9,7 +9,8 @@
 // (src/uma_qmoe/native_backend.py:530-543) with a stable counting sort: per
 // 64-route chunk, eight wave ballots give every lane the mask of lanes holding
 // the same expert id, so ranks come from one popcount and no comparison sort
-// is needed (one workgroup up to 3072 routes, one wavefront beyond).
+// is needed (one wavefront up to 64 routes, one workgroup up to 3072, a
+// workgroup per 1024 or more routes beyond).
 #include "uqm_route.h"
 
 namespace uqm {
@@ -152,6 +153,30 @@ __device__ __forceinline__ int load_route_id(const int32_t* route_expert, const 
   return valid ? static_cast<int>(id) : 0;
 }
 
+// Exclusive offsets of the experts into start[0..255] (LDS) from the counts
+// cnt[0..255] (one wavefront).
+__device__ void expert_starts(const int* cnt, int* start, int lane) {
+  int c4[4];
+  int local = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    c4[i] = cnt[4 * lane + i];
+    local += c4[i];
+  }
+  int incl = local;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(incl, o, kWave);
+    if (lane >= o) incl += v;
+  }
+  int pre = incl - local;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    start[4 * lane + i] = pre;
+    pre += c4[i];
+  }
+}
+
 // Per-expert tables from the counts cnt[0..255] (one wavefront): exclusive
 // offsets into start[] (LDS) and expert_offsets[E+1], the route tiles (when
 // tile_tokens > 0) and the compact list of experts that have routes.
@@ -240,7 +265,7 @@ __device__ __forceinline__ uint64_t same_id_lanes(int id, bool valid, int nbits)
   return eq;
 }
 
-// One wavefront; E <= 256. Any number of routes.
+// One wavefront, at most 64 routes; E <= 256.
 __global__ __launch_bounds__(64) void route_permute_kernel(const int32_t* __restrict__ route_expert,
                                                            const int64_t* __restrict__ indices64, int64_t n,
                                                            int E, int32_t* __restrict__ route_order,
@@ -252,39 +277,25 @@ __global__ __launch_bounds__(64) void route_permute_kernel(const int32_t* __rest
                                                            int32_t* __restrict__ tiles,
                                                            int32_t* __restrict__ tile_count) {
   __shared__ int cnt[256];
-  __shared__ int run[256];
+  __shared__ int start[256];
   const int lane = threadIdx.x;
   for (int e = lane; e < 256; e += 64) cnt[e] = 0;
   __syncthreads();
-
-  for (int64_t base = 0; base < n; base += 64) {
-    bool valid;
-    const int id = load_route_id(route_expert, indices64, base + lane, n, E, valid);
-    if (valid) atomicAdd(&cnt[id], 1);
-  }
-  __syncthreads();
-  expert_tables(cnt, run, lane, E, expert_offsets, offsets64, tile_tokens, tiles, tile_count, active_experts,
-                active_count);
-  __syncthreads();
-
   int nbits = 1;
   while ((1 << nbits) < E) ++nbits;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  for (int64_t base = 0; base < n; base += 64) {
-    bool valid;
-    const int id = load_route_id(route_expert, indices64, base + lane, n, E, valid);
-    const uint64_t eq = same_id_lanes(id, valid, nbits);
-    const int rank = __popcll(eq & lt);
-    int start = 0;
-    if (valid) start = run[id];
-    __syncthreads();
-    if (valid) {
-      const int pos = start + rank;
-      route_order[pos] = static_cast<int32_t>(base + lane);
-      if (order64 != nullptr) order64[pos] = base + lane;
-      if ((eq & lt) == 0) run[id] = start + __popcll(eq);
-    }
-    __syncthreads();
+  bool valid;
+  const int id = load_route_id(route_expert, indices64, lane, n, E, valid);
+  const uint64_t eq = same_id_lanes(id, valid, nbits);
+  if (valid && (eq & lt) == 0) cnt[id] = __popcll(eq);
+  __syncthreads();
+  expert_tables(cnt, start, lane, E, expert_offsets, offsets64, tile_tokens, tiles, tile_count, active_experts,
+                active_count);
+  __syncthreads();
+  if (valid) {
+    const int pos = start[id] + __popcll(eq & lt);
+    route_order[pos] = lane;
+    if (order64 != nullptr) order64[pos] = lane;
   }
 }
 
@@ -292,8 +303,7 @@ __global__ __launch_bounds__(64) void route_permute_kernel(const int32_t* __rest
 // routes are cut into 64-route chunks; every chunk's per-expert counts go to
 // an LDS histogram (ballot matching gives each route its rank inside its
 // chunk), a scan over the chunks per expert turns them into chunk bases, and
-// each route lands at offset[e] + base[chunk][e] + rank. Same stable order
-// as the one-wave kernel.
+// each route lands at offset[e] + base[chunk][e] + rank.
 constexpr int kPermuteMaxRoutes = 3072;
 constexpr int kPermuteWaves = 16;
 
@@ -381,6 +391,89 @@ __global__ __launch_bounds__(64 * kPermuteWaves) void route_permute_wg_kernel(
              offsets64, tile_tokens, tiles, tile_count);
 }
 
+// More than kPermuteMaxRoutes routes: workgroup b places the routes of segment
+// b (seg routes, a multiple of 1024). It needs, per expert, the routes before
+// its segment and the total; every workgroup counts all n ids itself (two LDS
+// counter rows, one atomic per route), so nothing is exchanged between
+// workgroups and one launch does. The counting is what bounds it: n / 64
+// wave-wide LDS atomics per workgroup, against n / 64 dependent trips of a
+// single wavefront before (3996 routes of 60 experts 8.6 vs 90 us, 32760
+// routes of 64 experts 17.7 vs 444 us, kernel trace). Then as above, 1024
+// routes at a time.
+__global__ __launch_bounds__(64 * kPermuteWaves) void route_permute_blocks_kernel(
+    const int32_t* __restrict__ route_expert, const int64_t* __restrict__ indices64, int64_t n, int64_t seg, int E,
+    int32_t* __restrict__ route_order, int32_t* __restrict__ expert_offsets, int32_t* __restrict__ active_experts,
+    int32_t* __restrict__ active_count, int64_t* __restrict__ order64, int64_t* __restrict__ offsets64,
+    int tile_tokens, int32_t* __restrict__ tiles, int32_t* __restrict__ tile_count) {
+  constexpr int kThreads = 64 * kPermuteWaves;
+  constexpr int kBatch = 8;  // ids in flight per thread while counting
+  __shared__ int hist[kPermuteWaves][256];
+  __shared__ int cnt[2][256];  // routes before the segment; from it on
+  __shared__ int base[256];
+  const int wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int64_t beg = blockIdx.x * seg;
+  const int64_t end = beg + seg < n ? beg + seg : n;
+  for (int i = threadIdx.x; i < 512; i += kThreads) (&cnt[0][0])[i] = 0;
+  __syncthreads();
+  for (int64_t r0 = 0; r0 < n; r0 += static_cast<int64_t>(kBatch) * kThreads) {
+    int ids[kBatch];
+    bool oks[kBatch];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j)
+      ids[j] = load_route_id(route_expert, indices64, r0 + j * kThreads + threadIdx.x, n, E, oks[j]);
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      const int64_t r = r0 + j * kThreads + threadIdx.x;
+      if (oks[j]) atomicAdd(&cnt[r < beg ? 0 : 1][ids[j]], 1);
+    }
+  }
+  __syncthreads();
+  // totals per expert into hist[0], then the experts' starts
+  if (threadIdx.x < 256) hist[0][threadIdx.x] = cnt[0][threadIdx.x] + cnt[1][threadIdx.x];
+  __syncthreads();
+  if (wave == 0) {
+    if (blockIdx.x == 0)
+      expert_tables(hist[0], base, lane, E, expert_offsets, offsets64, tile_tokens, tiles, tile_count, active_experts,
+                    active_count);
+    else
+      expert_starts(hist[0], base, lane);
+  }
+  __syncthreads();
+  if (threadIdx.x < 256) base[threadIdx.x] += cnt[0][threadIdx.x];
+
+  int nbits = 1;
+  while ((1 << nbits) < E) ++nbits;
+  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  for (int64_t c0 = beg; c0 < end; c0 += kThreads) {
+    for (int i = threadIdx.x; i < kPermuteWaves * 256; i += kThreads) (&hist[0][0])[i] = 0;
+    __syncthreads();
+    const int64_t r = c0 + threadIdx.x;
+    bool valid;
+    const int id = load_route_id(route_expert, indices64, r, end, E, valid);
+    const uint64_t eq = same_id_lanes(id, valid, nbits);
+    if (valid && (eq & lt) == 0) hist[wave][id] = __popcll(eq);
+    __syncthreads();
+    if (threadIdx.x < 256) {
+      int run = base[threadIdx.x];
+#pragma unroll
+      for (int ch = 0; ch < kPermuteWaves; ++ch) {
+        const int v = hist[ch][threadIdx.x];
+        hist[ch][threadIdx.x] = run;
+        run += v;
+      }
+      base[threadIdx.x] = run;
+    }
+    __syncthreads();
+    if (valid) {
+      const int pos = hist[wave][id] + __popcll(eq & lt);
+      route_order[pos] = static_cast<int32_t>(r);
+      if (order64 != nullptr) order64[pos] = r;
+    }
+    __syncthreads();
+  }
+}
+
 // Top-k and permutation in one launch (up to kPermuteMaxRoutes routes): one
 // token per wavefront. The route ids are written with device-coherent stores;
 // once they have completed, every workgroup counts itself done on a
@@ -433,15 +526,26 @@ hipError_t launch_route_permute(const int32_t* route_expert, const int64_t* indi
                                 int64_t E, const RouteTables& rt, int64_t* order64, int64_t* offsets64,
                                 int tile_tokens, hipStream_t stream) {
   if (tile_tokens > 0 && (rt.tiles == nullptr || rt.tile_count == nullptr)) return hipErrorInvalidValue;
-  if (n_routes > 64 && n_routes <= kPermuteMaxRoutes)
+  if (n_routes > kPermuteMaxRoutes) {
+    // 1024 routes (one pass of the ranking) per workgroup; longer segments
+    // only where that would be more than 64 workgroups, all of which read all
+    // the ids
+    int64_t seg = 1024;
+    while ((n_routes + seg - 1) / seg > 64) seg *= 2;
+    hipLaunchKernelGGL(route_permute_blocks_kernel, dim3(static_cast<unsigned>((n_routes + seg - 1) / seg)),
+                       dim3(64 * kPermuteWaves), 0, stream, route_expert, indices64, n_routes, seg,
+                       static_cast<int>(E), rt.route_order, rt.expert_offsets, rt.active_experts, rt.active_count,
+                       order64, offsets64, tile_tokens, rt.tiles, rt.tile_count);
+  } else if (n_routes > 64) {
     hipLaunchKernelGGL(route_permute_wg_kernel, dim3(1), dim3(64 * kPermuteWaves), permute_lds_bytes(n_routes), stream,
                        route_expert, indices64,
                        n_routes, static_cast<int>(E), rt.route_order, rt.expert_offsets, rt.active_experts,
                        rt.active_count, order64, offsets64, tile_tokens, rt.tiles, rt.tile_count);
-  else
+  } else {
     hipLaunchKernelGGL(route_permute_kernel, dim3(1), dim3(64), 0, stream, route_expert, indices64, n_routes,
                        static_cast<int>(E), rt.route_order, rt.expert_offsets, rt.active_experts, rt.active_count,
                        order64, offsets64, tile_tokens, rt.tiles, rt.tile_count);
+  }
   return hipGetLastError();
 }
 
