@@ -1,0 +1,112 @@
+"""GPU parity of the large-tile grouped GEMM (many routes per expert) against
+the CPU oracle.
+
+Its outputs are BF16 roundings of FP32 sums over BF16-rounded SiLU products, as
+the oracle's, so both differ from the exact value by about 2^-9 per rounding:
+rel-L2 <= 1e-2 and max-abs <= 2e-2, the bounds of every routed path."""
+
+from __future__ import annotations
+
+from dataclasses import replace
+
+import pytest
+import torch
+
+from oracle import moe as om
+from test_gpu_mfma import DEV, close, mfma_on, note, to_dev  # noqa: F401
+from uma_qmoe_amd import synthetic as syn
+
+pytestmark = pytest.mark.gpu
+
+# Routes per expert: one route, both sides of a 16-route step (every tile size
+# of the kernel), the largest single tile, the first split, several tiles, none.
+COUNTS = [1, 15, 16, 17, 32, 33, 49, 64, 65, 81, 97, 112, 113, 128, 129, 144, 145, 289, 0, 433]
+# (H, I): K groups even and odd in either projection, from the smallest K on
+SHAPES = [(640, 384), (256, 640), (512, 256), (1152, 896)]
+
+
+def skewed_routes(counts, seed):
+    """idx [T, 1] with counts[e] routes of expert e, in random order."""
+    g = torch.Generator().manual_seed(seed)
+    ids = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))
+    ids = ids[torch.randperm(ids.numel(), generator=g)]
+    return ids.view(-1, 1), torch.rand(ids.numel(), 1, generator=g).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("encoding", ["q4_group128", "q8_group128", "bf16_le"])
+@pytest.mark.parametrize("hidden,inter", SHAPES)
+def test_tile_sizes_against_oracle(mfma_on, encoding, hidden, inter):  # noqa: F811
+    shape = syn.MoEShape("prefill", hidden, len(COUNTS), 1, inter, encoding=encoding)
+    note(f"prefill {encoding} H={hidden} I={inter}")
+    layer = syn.build_experts(shape, seed=hidden)
+    idx, w = skewed_routes(COUNTS, inter)
+    assert idx.numel() / len(COUNTS) >= 44  # the large-tile kernel's range for every encoding
+    x = syn.hidden_states(shape, idx.shape[0], seed=3)
+    got = mfma_on.moe_forward(to_dev(layer), x.to(DEV), idx.to(DEV), w.to(DEV))
+    ref = om.streaming_reference(x, idx, w, 0, syn.DeviceLayerReader({0: layer}), num_experts=len(COUNTS))
+    close(got, ref, f"{encoding} H={hidden} I={inter}")
+
+
+@pytest.mark.parametrize("encoding", ["q4_group128", "q8_group128"])
+def test_wide_scale_groups_and_dropped_routes(mfma_on, encoding):  # noqa: F811
+    """Scale groups of 256 elements (two K groups share a scale), top-2 routes
+    with ids out of range."""
+    shape = syn.MoEShape("prefill_g256", 512, 5, 2, 256, encoding=encoding, group_size=256)
+    note(f"prefill group 256 {encoding}")
+    layer = syn.build_experts(shape, seed=9)
+    g = torch.Generator().manual_seed(4)
+    idx = torch.stack([torch.randperm(5, generator=g)[:2] for _ in range(333)])
+    w = torch.rand(333, 2, generator=g).to(torch.bfloat16)
+    x = syn.hidden_states(shape, 333, seed=5)
+    dropped = idx.clone()
+    dropped[::5, 1] = -1
+    dropped[1::7, 0] = 5
+    w_ref = w.clone()
+    w_ref[::5, 1] = 0
+    w_ref[1::7, 0] = 0
+    got = mfma_on.moe_forward(to_dev(layer), x.to(DEV), dropped.to(DEV), w.to(DEV))
+    ref = om.streaming_reference(x, idx, w_ref, 0, syn.DeviceLayerReader({0: layer}), num_experts=5)
+    close(got, ref, f"group 256 {encoding}")
+
+
+def test_infinities_and_nan_stay_in_their_token(mfma_on):  # noqa: F811
+    """Non-finite activations poison their own token's output and no other."""
+    shape = syn.MoEShape("prefill_nan", 256, 2, 1, 256, encoding="q4_group128")
+    note("prefill non-finite")
+    layer = to_dev(syn.build_experts(shape, seed=2))
+    t = 150
+    idx = (torch.arange(t) % 2).view(-1, 1)
+    w = torch.ones(t, 1, dtype=torch.bfloat16)
+    x = syn.hidden_states(shape, t, seed=6)
+    clean = mfma_on.moe_forward(layer, x.to(DEV), idx.to(DEV), w.to(DEV)).cpu()
+    bad = x.clone()
+    bad[0, 3] = float("nan")  # token 0 pads expert 0's last tile
+    bad[7, 9] = float("inf")
+    out = mfma_on.moe_forward(layer, bad.to(DEV), idx.to(DEV), w.to(DEV)).cpu()
+    keep = torch.ones(t, dtype=torch.bool)
+    keep[[0, 7]] = False
+    assert torch.equal(out[keep], clean[keep])
+    assert out[0].isnan().all() and not out[7].isfinite().all()
+
+
+def test_block_replays_from_a_graph(mfma_on):  # noqa: F811
+    """A whole block on the large tiles, captured and replayed with eager work
+    in between, equals the eager call bit for bit."""
+    shape = replace(syn.C2, num_experts=8, intermediate=384, shared_intermediate=512)
+    note("prefill graph")
+    ext = mfma_on
+    layer = syn.build_experts(shape, device=DEV)
+    dense = syn.build_dense(shape, device=DEV)
+    x = syn.hidden_states(shape, 900, device=DEV)  # 3600 routes, 450 per expert
+    ws = ext.new_workspace(DEV, 900, shape.hidden, shape.intermediate, shape.shared_intermediate, 8, shape.top_k)
+    ref = ext.moe_layer(layer, dense, x, shape.top_k, workspace=ws)[0].clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        res = ext.moe_layer(layer, dense, x, shape.top_k, workspace=ws)[0]
+    for _ in range(3):
+        res.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(res, ref)
+        ext.moe_layer(layer, dense, x, shape.top_k, workspace=ws)

@@ -13,6 +13,7 @@
 #include "../../include/uma_qmoe_hip.h"
 #include "uqm_dense.h"
 #include "uqm_internal.h"
+#include "uqm_prefill.h"
 #include "uqm_route.h"
 
 namespace {
@@ -235,16 +236,32 @@ bool routed_uses_stream(const uqm_expert_weights* w) {
          uqm::stream_supported(w->encoding, w->intermediate_size, w->group_size);
 }
 
+// Whether the routed projections of T tokens take the large-tile kernel
+// (uqm_prefill.hip): from 44 routes per active expert on average for Q4 and
+// from 30 for Q8 and BF16. Its items dequantise a row once for up to 144
+// routes; the smaller tiles of uqm_mfma.hip waste less below. Measured, large
+// tiles against small (us per call): Q4 Qwen block 204 vs 200 at 43 routes and
+// 242 vs 306 at 68, Q4 128 experts Zipf 169 vs 173 at 44; Q8 Qwen block 218 vs
+// 231 at 32, 214 vs 206 at 29; BF16 285 vs 300 at 32, 283 vs 282 at 29.
+bool routed_uses_prefill(const uqm_expert_weights* w, int64_t T, int64_t R, double mean) {
+  const int64_t min_t = g_opt_mfma_min_tokens.load(std::memory_order_relaxed);
+  if (min_t <= 0 || T < min_t || mean < (w->encoding == UQM_Q4 ? 44.0 : 30.0)) return false;
+  const int64_t H = w->hidden_size, I = w->intermediate_size;
+  return uqm::prefill_supported(w->encoding, I, H, w->group_size, T, H) &&
+         uqm::prefill_supported(w->encoding, H, I, w->group_size, R, I);
+}
+
 // Route tile size the routed MFMA path uses (0 = GEMV path). From 16 routes
 // per expert on average, 32-route tiles: measured faster than 16 (c5: 80 vs
 // 105 us) and than 64 (c4: 247 vs 271 us), whose 4-wave items take longer per
 // weight byte.
 int routed_tile_tokens(const uqm_expert_weights* w, int64_t T, int64_t k) {
-  if (!routed_uses_mfma(w, T)) return 0;
   const int64_t R = T * k;
   const int64_t active = R < w->num_experts ? R : w->num_experts;
   const double mean = static_cast<double>(R) / static_cast<double>(active);
   if (routed_uses_stream(w) && R <= g_opt_stream_max_routes.load(std::memory_order_relaxed)) return 0;
+  if (routed_uses_prefill(w, T, R, mean)) return uqm::kPrefillTileTokens;
+  if (!routed_uses_mfma(w, T)) return 0;
   // 48-route tiles when most experts would otherwise take a second, nearly
   // empty 32-route tile (every tile costs a full pass over the expert's rows)
   // and both Q4 projections run 128-row items (the only kernels built for them)
@@ -434,8 +451,11 @@ int run_routed(const uqm_expert_weights* w, const uint16_t* hidden, int64_t T, i
     // many tiles (c5) share their rows with tiles fastest (53 vs 60 MB for 40)
     g.order = kOrderAuto;
     g.active_count = at<int32_t>(ws, L.counters);
+    const bool prefill = tile_tokens == kPrefillTileTokens;
     const MfmaPlan pg = plan_mfma(w->encoding, 2, I, H, nb, active, cus, 1);
-    int rc = hip_check(launch_expert_mfma(w->encoding, 2, g, pg.nb, pg.kw, pg.mw, cus, stream), "gate/up MFMA launch");
+    int rc = hip_check(prefill ? launch_prefill_mfma(w->encoding, 2, kModeSilu, g, stream)
+                               : launch_expert_mfma(w->encoding, 2, g, pg.nb, pg.kw, pg.mw, cus, stream),
+                       "gate/up MFMA launch");
     if (rc) return rc;
     MfmaArgs d = g;
     d.w[0] = static_cast<const uint8_t*>(w->down);
@@ -451,6 +471,8 @@ int run_routed(const uqm_expert_weights* w, const uint16_t* hidden, int64_t T, i
     d.ldo = H;
     d.part_stride = R * H;
     d.order = kOrderRowFastest;
+    if (prefill)
+      return hip_check(launch_prefill_mfma(w->encoding, 1, kModeF32, d, stream), "down MFMA launch");
     const MfmaPlan pd = plan_mfma(w->encoding, 1, H, I, nb, active, cus, T > 1 ? kMaxSplit : 1);
     d.ksplit = pd.ksplit;
     *parts = pd.ksplit;

@@ -1,0 +1,479 @@
+// Expert-grouped GEMM for calls with many routes per expert (long prefill).
+//
+// Covers the same projections as uqm_mfma.hip (the reference's prefill kernels,
+// src/uma_qmoe/native/packed_q4_kernel.cu:560-776 for Q4, :781-1099 for Q8, and
+// its BF16 grouped_mm path, src/uma_qmoe/native_backend.py:958-1005).
+//
+// What bounds uqm_mfma.hip there is its MMA waves' instruction stream: a route
+// tile of 32 means that every 32 routes dequantise the expert's rows again, and
+// an offset-binary weight needs the activation sums (one more MFMA per two).
+// Here one workgroup of 4 waves takes 128 weight rows (gate/up: 64 of each) and
+// up to 144 routes, each wave 32 rows and all the routes:
+//   * weights go straight from global memory to the wave that uses them (no
+//     row is shared between waves), one 128-element group ahead, and become
+//     signed bf16 integers in registers: v_cvt_off_f32_i4 (q / 16) and
+//     v_cvt_f32_i32 with a sign-extended byte are exact in bf16, so the MFMA
+//     sums x * q directly and needs no activation sums; per 128-element group
+//     acc += scale * sum in FP32. That is 104 conversions per group and 8 FMAs
+//     per 16-route tile against 8 MFMAs per tile: at 9 tiles 2.4 VALU
+//     instructions per MFMA, spread evenly between them (the next group is
+//     converted while this one's MFMAs run, each tile's B operands are read
+//     during the tile before, its sums folded during the one after);
+//   * activations come through LDS (global_load_lds, 16 bytes per lane, one
+//     128-element group of all routes per stage) in a ring of 2 to 4 stages,
+//     and the group's scales with them, so that a lane reads the scales of its
+//     4 rows as one vector;
+//   * an expert's routes are split evenly (route_tile_step), and the loop is
+//     compiled for every tile size from 1 to 9 sixteens, so that padding stays
+//     below 16 routes per tile;
+//   * one work item per workgroup and two workgroups per CU (72 KB of ring, at
+//     most 256 VGPRs): the hardware dispatcher balances items of different
+//     sizes, and one workgroup's start and end run under the other's MFMAs.
+// What bounds it: MFMA and VALU time, which add up on a SIMD (counters at the
+// first size below: 37% and 40% of the cycles, 20% of the wave time waiting).
+// Measured (kernel trace, us, large tiles against uqm_mfma.hip's 32 routes):
+// OLMoE shapes, 4095 tokens (512 routes per expert), Q4: gate/up 325 vs 859,
+// down 214 vs 458; Qwen shapes, routed experts alone: Q4 2048 tokens 168 + 92
+// (233 + 141 beside the shared expert), Q8 999 tokens 137 + 69 (215 + 102),
+// BF16 1535 tokens 203 + 101 (344 + 169; 3.4 TB/s of weights).
+//
+// MFMA operand layout (v_mfma_f32_16x16x32_bf16): A lane l holds row l%16 and
+// K-slice 8*(l/16)..+7; B lane l holds token l%16, same K-slice; D lane l
+// holds token l%16, rows 4*(l/16)+i. The K elements of a step follow the order
+// of a lane's 16-byte weight loads, the same for A and B.
+#include "uqm_prefill.h"
+
+#include <type_traits>
+
+namespace uqm {
+namespace {
+
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void prefill_lds_t;
+
+constexpr int kWaves = 4;
+constexpr int kThreads = 64 * kWaves;
+constexpr int kRowBytes = 256;                  // one staged activation row: 128 bf16
+constexpr int kTileBytes = 16 * kRowBytes;      // 16 routes of one stage
+constexpr int kMaxTT = kPrefillTileTokens / 16;  // 16-route tiles per item
+constexpr int kRingTiles = 18;                  // 72 KB
+constexpr int kMaxStages = 4;
+
+// Stages of the ring for items of TT tiles: small items run through a stage
+// in well under a microsecond and need more of them in flight.
+constexpr int stages_for(int tt) { return kRingTiles / tt < kMaxStages ? kRingTiles / tt : kMaxStages; }
+
+constexpr int kScaleOff = kRingTiles * kTileBytes;             // [stage][128] floats
+constexpr int kRouteOff = kScaleOff + kMaxStages * 128 * 4;    // [kPrefillTileTokens] route ids
+constexpr int kSourceOff = kRouteOff + kPrefillTileTokens * 4;  // [kPrefillTileTokens] activation rows
+constexpr int kLdsBytes = kSourceOff + kPrefillTileTokens * 4;
+static_assert(2 * kLdsBytes <= 160 * 1024, "two workgroups per CU");
+
+template <int ENC>
+struct PEnc;
+template <>
+struct PEnc<kQ4> {
+  static constexpr int kLoads = 1;         // 16-byte loads per lane, 16-row tile and 128-element group
+  static constexpr int kGroupBytes = 64;   // bytes of one row's group
+};
+template <>
+struct PEnc<kQ8> {
+  static constexpr int kLoads = 2;
+  static constexpr int kGroupBytes = 128;
+};
+template <>
+struct PEnc<kBF16> {
+  static constexpr int kLoads = 4;
+  static constexpr int kGroupBytes = 256;
+};
+
+__device__ __forceinline__ uint32_t dword_of(const uint4& v, int i) {
+  return i == 0 ? v.x : (i == 1 ? v.y : (i == 2 ? v.z : v.w));
+}
+
+// bf16 pair of two floats that are exact in bf16.
+__device__ __forceinline__ uint32_t exact_pair(float lo, float hi) {
+  return perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+
+// Dword i (a bf16 pair) of the A operand (8 weights) of K-step S of a group
+// from the lane's 16-byte loads:
+//   Q4: dword S = elements 32q+8S .. +7, as q / 16
+//   Q8: load S/2, dwords 2(S%2), 2(S%2)+1 = elements 64(S/2)+16q+8(S%2) .. +7
+//   BF16: load S = elements 32S+8q .. +7
+template <int ENC>
+__device__ __forceinline__ uint32_t weight_pair(const uint4 (&v)[PEnc<ENC>::kLoads], int S, int i) {
+  if constexpr (ENC == kQ4) {
+    const uint32_t w = dword_of(v[0], S);
+    uint32_t h = w >> 4;  // high nibble of byte i at bits 3:0 of its byte i
+    asm("" : "+v"(h));    // (one shift per dword: the conversions select their byte)
+    return exact_pair(__builtin_amdgcn_cvt_off_f32_i4((w >> (8 * i)) & 0xFFu),
+                      __builtin_amdgcn_cvt_off_f32_i4((h >> (8 * i)) & 0xFFu));
+  } else if constexpr (ENC == kQ8) {
+    const uint32_t d = dword_of(v[S >> 1], 2 * (S & 1) + (i >> 1)) >> (16 * (i & 1));
+    return exact_pair(static_cast<float>(static_cast<int8_t>(d)), static_cast<float>(static_cast<int8_t>(d >> 8)));
+  } else {
+    return dword_of(v[S], i);
+  }
+}
+
+// 16-byte slot (8 elements, within a group) of the B operand of K-step S for
+// lane quadrant q, matching weight_frag's order.
+template <int ENC>
+__device__ __forceinline__ int x_slot(int q, int S) {
+  if constexpr (ENC == kQ4) return 4 * q + S;
+  else if constexpr (ENC == kQ8) return 8 * (S >> 1) + 2 * q + (S & 1);
+  else return 4 * S + q;
+}
+
+// g / (1 + exp(-g)): the reciprocal refined by one Newton step, as accurate as
+// the divide at half its instructions. Where exp overflows (g below -88) the
+// reciprocal is 0 and the step's NaN becomes 1, so the result is -0 as with
+// the divide (NaN for -inf).
+__device__ __forceinline__ float silu_newton(float g) {
+  const float d = 1.0f + __expf(-g);
+  const float r = __builtin_amdgcn_rcpf(d);
+  return g * fmaf(fminf(fmaf(-d, r, 1.0f), 1.0f), r, r);
+}
+
+// s_waitcnt with only vmcnt limited (gfx9 encoding: vmcnt bits 3:0 and 15:14).
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  static_assert(N >= 0 && N <= 63, "vmcnt is 6 bits");
+  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
+
+// This wave's LDS reads complete, then the workgroup barrier (loads into LDS
+// are waited for separately, by stage).
+__device__ __forceinline__ void stage_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), vmcnt and expcnt unlimited
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// 16 or 4 bytes per lane from global memory into LDS at a wave-uniform LDS
+// byte address (lane l's bytes at lds_addr + 16 l or + 4 l).
+__device__ __forceinline__ void dma16(const void* src, uint32_t lds_addr) {
+  __builtin_amdgcn_global_load_lds(src, reinterpret_cast<prefill_lds_t*>(static_cast<uintptr_t>(lds_addr)), 16, 0, 0);
+}
+__device__ __forceinline__ void dma4(const void* src, uint32_t lds_addr) {
+  __builtin_amdgcn_global_load_lds(src, reinterpret_cast<prefill_lds_t*>(static_cast<uintptr_t>(lds_addr)), 4, 0, 0);
+}
+
+// One work item of TT 16-route tiles: rows of row block rb of `expert`, the
+// nt <= 16 TT routes listed in LDS.
+template <int ENC, int NMAT, int MODE, int TT>
+__device__ __forceinline__ void run_item(const MfmaArgs& a, unsigned char* lds, int expert, int rb, int nt) {
+  using E = PEnc<ENC>;
+  constexpr bool kScaled = ENC != kBF16;
+  constexpr int L = E::kLoads;
+  constexpr int D = stages_for(TT);
+  constexpr int kStageBytes = TT * kTileBytes;
+  constexpr int kPerStage = TT + (kScaled ? 1 : 0);  // loads into LDS per wave and stage
+  static_assert((D - 2) * kPerStage <= 63, "outstanding loads must fit vmcnt");
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int q = lane >> 4, t16 = lane & 15;
+  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((prefill_lds_t*)(lds)));
+  const int S = static_cast<int>(a.K / 128);
+  const int rows = static_cast<int>(a.rows);
+  const uint32_t row_bytes = static_cast<uint32_t>(S) * E::kGroupBytes;
+  const int* ids = reinterpret_cast<const int*>(lds + kRouteOff);
+  const int* srcs = reinterpret_cast<const int*>(lds + kSourceOff);
+
+  // ---- sources: weight rows, activation rows, scales ----
+  const uint8_t* wbase[2];
+  uint32_t woff[2];
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt) {
+    int row = NMAT == 2 ? rb * 64 + 16 * wave + t16 : rb * 128 + 32 * wave + 16 * mt + t16;
+    row = min(row, rows - 1);  // padding rows of the last block repeat the last row
+    wbase[mt] = a.w[NMAT == 2 ? mt : 0] + static_cast<int64_t>(expert) * rows * row_bytes;
+    woff[mt] = static_cast<uint32_t>(row) * row_bytes + 16 * q;
+  }
+  uint32_t xoff[TT];
+#pragma unroll
+  for (int j = 0; j < TT; ++j) {
+    const int r = 16 * j + 4 * wave + q;  // staged row this lane fills, at position t16
+    const int u = t16 ^ (r & 15);
+    xoff[j] = static_cast<uint32_t>(srcs[r]) * static_cast<uint32_t>(a.ldx * 2) + 16 * x_slot<ENC>(u & 3, u >> 2);
+  }
+  const uint8_t* const x = reinterpret_cast<const uint8_t*>(a.x);
+  const float* ssrc = nullptr;
+  int gdiv = 1;
+  if constexpr (kScaled) {
+    const int G = static_cast<int>(a.K / a.group);
+    gdiv = static_cast<int>(a.group / 128);
+    int row = NMAT == 2 ? rb * 64 + lane : rb * 128 + 64 * (wave & 1) + lane;
+    row = min(row, rows - 1);
+    ssrc = a.s[NMAT == 2 ? wave & 1 : 0] + static_cast<int64_t>(expert) * a.scales_per_expert +
+           static_cast<int64_t>(row) * G;
+  }
+
+  auto issue = [&](int g, int slot) {
+    const uint32_t buf = __builtin_amdgcn_readfirstlane(lds_base + static_cast<uint32_t>(slot * kStageBytes));
+    const uint8_t* xg = x + static_cast<int64_t>(g) * kRowBytes;
+#pragma unroll
+    for (int j = 0; j < TT; ++j) {
+      uint32_t o = xoff[j];
+      asm("" : "+v"(o));  // (extended to 64 bits by the load itself, not kept extended)
+      dma16(xg + o, buf + (16 * j + 4 * wave) * kRowBytes);
+    }
+    if constexpr (kScaled) {
+      // waves 2 and 3 repeat what waves 0 and 1 load, so that every wave waits
+      // for the same number of loads
+      dma4(ssrc + g / gdiv, __builtin_amdgcn_readfirstlane(lds_base + kScaleOff + slot * 512 + (wave & 1) * 256));
+    }
+  };
+  auto load_weights = [&](int g, uint4 (&v)[2][L]) {
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int u = 0; u < L; ++u) v[mt][u] = ldg16(wbase[mt] + (woff[mt] + static_cast<uint32_t>(g * E::kGroupBytes + 64 * u)));
+  };
+
+  f32x4_t acc[2][TT];
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) acc[mt][tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  uint32_t xo[4];  // LDS byte (within a 16-route tile) of this lane's B operand of each K-step
+#pragma unroll
+  for (int s = 0; s < 4; ++s) xo[s] = static_cast<uint32_t>(t16 * kRowBytes + (((q + 4 * s) ^ t16) << 4));
+  const int srow = NMAT == 2 ? 16 * wave + 4 * q : 32 * wave + 4 * q;
+
+  // Waits until the next stage is resident: of this wave's loads into LDS only
+  // those of the D - 2 stages after it may be in flight. (Loads complete in
+  // issue order; weight loads in between only make the wait stricter.)
+  auto wait_next = [&]() { wait_loads<(D - 2) * kPerStage>(); };
+
+  struct Weights {
+    u32x4_t f[2][4];  // A operands of a group: [16-row tile][K-step] (Q4, Q8)
+  };
+  struct Raw {
+    uint4 v[2][L];
+  };
+  auto convert = [&](const Raw& r, Weights& w, int unit) {  // pair `unit` (0..31) of a group's operands
+    const int mt = unit & 1, S_ = unit >> 3, i = (unit >> 1) & 3;
+    w.f[mt][S_][i] = weight_pair<ENC>(r.v[mt], S_, i);
+  };
+  int slot = 0;
+  // One group (stage). Q4, Q8: its MFMAs from `w`, while `r` (the next group's
+  // bytes) becomes `wn` and the bytes of the group after it are loaded into
+  // `rn`. BF16: its MFMAs from `r`, while the next group's are loaded into `rn`.
+  auto group = [&](int g, const Weights& w, const Raw& r, Weights& wn, Raw& rn) {
+    load_weights(min(g + (kScaled ? 2 : 1), S - 1), rn.v);
+    __builtin_amdgcn_sched_barrier(0);
+    // (past the last stage the last one is loaded again, into a buffer nothing
+    // reads: a branch here would split the group's code and let the compiler
+    // move its arithmetic out of it)
+    issue(min(g + D - 1, S - 1), slot == 0 ? D - 1 : slot - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    const unsigned char* buf = lds + slot * kStageBytes;
+    f32x4_t sc[2];
+    if constexpr (kScaled) {
+      const float* sl = reinterpret_cast<const float*>(lds + kScaleOff + slot * 512) + srow;
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) sc[mt] = *reinterpret_cast<const f32x4_t*>(sl + (NMAT == 2 ? 64 : 16) * mt);
+    }
+    bf16x8_t b[2][4];
+    f32x4_t d[2][2];
+    auto read = [&](int tt) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) b[tt & 1][s] = *reinterpret_cast<const bf16x8_t*>(buf + xo[s] + tt * kTileBytes);
+    };
+    auto fold = [&](int tt) {  // acc += scale * (sums over the group)
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[mt][tt][e] = fmaf(sc[mt][e], d[tt & 1][mt][e], acc[mt][tt][e]);
+    };
+    read(0);
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+      if (tt + 1 < TT) read(tt + 1);
+      if constexpr (kScaled) {
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) d[tt & 1][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+          f32x4_t& c = kScaled ? d[tt & 1][mt] : acc[mt][tt];
+          bf16x8_t af;
+          if constexpr (kScaled)
+            af = __builtin_bit_cast(bf16x8_t, w.f[mt][s]);
+          else
+            af = __builtin_bit_cast(bf16x8_t, r.v[mt][s]);
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, b[tt & 1][s], c, 0, 0, 0);
+        }
+      if constexpr (kScaled) {
+        if (tt > 0) fold(tt - 1);
+#pragma unroll
+        for (int unit = 32 * tt / TT; unit < 32 * (tt + 1) / TT; ++unit) convert(r, wn, unit);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (kScaled) fold(TT - 1);
+    wait_next();
+    stage_barrier();  // stage g consumed, stage g + 1 resident
+    slot = slot + 1 == D ? 0 : slot + 1;
+  };
+
+  Weights w0, w1;
+  Raw r0, r1;
+#pragma unroll
+  for (int g = 0; g < D - 1; ++g) issue(min(g, S - 1), g);
+  __builtin_amdgcn_sched_barrier(0);
+  load_weights(0, r0.v);
+  if constexpr (kScaled) {
+    load_weights(min(1, S - 1), r1.v);
+#pragma unroll
+    for (int unit = 0; unit < 32; ++unit) convert(r0, w0, unit);
+  }
+  wait_next();
+  stage_barrier();
+  Raw& ra = kScaled ? r1 : r0;
+  Raw& rz = kScaled ? r0 : r1;
+  int g = 0;
+  for (; g + 1 < S; g += 2) {
+    group(g, w0, ra, w1, rz);
+    group(g + 1, w1, rz, w0, ra);
+  }
+  if (g < S) group(g, w0, ra, w1, rz);
+  wait_loads<0>();  // no load into LDS outlives the workgroup
+
+  // ---- outputs ----
+#pragma unroll
+  for (int tt = 0; tt < TT; ++tt) {
+    const int tok = 16 * tt + t16;
+    if (tok >= nt) continue;
+    const int64_t at = static_cast<int64_t>(ids[tok]) * a.ldo;
+    constexpr float kUnit = ENC == kQ4 ? 16.f : 1.f;  // Q4 weights enter as q / 16
+    if constexpr (MODE == kModeSilu) {
+      const int r0 = rb * 64 + 16 * wave + 4 * q;
+      if (r0 >= rows) continue;
+      uint32_t h[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const uint32_t g2 = pack_bf16x2(kUnit * acc[0][tt][2 * e], kUnit * acc[0][tt][2 * e + 1]);
+        const uint32_t u2 = pack_bf16x2(kUnit * acc[1][tt][2 * e], kUnit * acc[1][tt][2 * e + 1]);
+        h[e] = pack_bf16x2(silu_newton(bf16lo(g2)) * bf16lo(u2), silu_newton(bf16hi(g2)) * bf16hi(u2));
+      }
+      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + at + r0) = make_uint2(h[0], h[1]);
+    } else {
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt) {
+        const int r0 = rb * 128 + 32 * wave + 16 * mt + 4 * q;
+        if (r0 >= rows) continue;
+        const f32x4_t v = acc[mt][tt] * kUnit;
+        if constexpr (MODE == kModeF32)
+          *reinterpret_cast<float4*>(static_cast<float*>(a.out) + at + r0) = make_float4(v[0], v[1], v[2], v[3]);
+        else
+          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + at + r0) =
+              make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+      }
+    }
+  }
+}
+
+}  // namespace
+
+// One work item per workgroup. The items (row blocks of a tile next to each
+// other, tiles in expert order) are split into 8 contiguous ranges, one per
+// XCD (blockIdx % 8), so that a tile's row blocks share its activations and an
+// expert's tiles share its rows in one XCD's L2.
+template <int ENC, int NMAT, int MODE>
+__global__ __launch_bounds__(kThreads, 2) void prefill_mfma_kernel(MfmaArgs a) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int n_tiles = a.tiles != nullptr ? *a.tile_count : a.tile_bound;
+  const int64_t n_items = static_cast<int64_t>(n_tiles) * a.row_blocks;
+  const int xcd = static_cast<int>(blockIdx.x & 7u);
+  const int64_t item = n_items * xcd / 8 + (blockIdx.x >> 3);
+  if (item >= n_items * (xcd + 1) / 8) return;  // uniform over the workgroup
+  const int tile = __builtin_amdgcn_readfirstlane(static_cast<int>(item / a.row_blocks));
+  const int rb = __builtin_amdgcn_readfirstlane(static_cast<int>(item % a.row_blocks));
+  int expert = 0, first, nt;
+  if (a.tiles != nullptr) {
+    expert = __builtin_amdgcn_readfirstlane(a.tiles[2 * tile]);
+    first = __builtin_amdgcn_readfirstlane(a.tiles[2 * tile + 1]);
+    const int beg = __builtin_amdgcn_readfirstlane(a.expert_offsets[expert]);
+    const int end = __builtin_amdgcn_readfirstlane(a.expert_offsets[expert + 1]);
+    nt = min(route_tile_step(end - beg, kPrefillTileTokens), end - first);
+  } else {
+    const int step = route_tile_step(a.n_routes, kPrefillTileTokens);
+    first = tile * step;
+    nt = min(step, a.n_routes - first);
+  }
+  int* ids = reinterpret_cast<int*>(lds + kRouteOff);
+  int* srcs = reinterpret_cast<int*>(lds + kSourceOff);
+  for (int i = threadIdx.x; i < kPrefillTileTokens; i += kThreads) {
+    int route = first + (i < nt ? i : 0);  // padding repeats the first route
+    if (a.route_order != nullptr) route = a.route_order[route];
+    ids[i] = route;
+    srcs[i] = route / a.x_div;
+  }
+  __syncthreads();
+  switch ((nt + 15) / 16) {
+    case 1: run_item<ENC, NMAT, MODE, 1>(a, lds, expert, rb, nt); break;
+    case 2: run_item<ENC, NMAT, MODE, 2>(a, lds, expert, rb, nt); break;
+    case 3: run_item<ENC, NMAT, MODE, 3>(a, lds, expert, rb, nt); break;
+    case 4: run_item<ENC, NMAT, MODE, 4>(a, lds, expert, rb, nt); break;
+    case 5: run_item<ENC, NMAT, MODE, 5>(a, lds, expert, rb, nt); break;
+    case 6: run_item<ENC, NMAT, MODE, 6>(a, lds, expert, rb, nt); break;
+    case 7: run_item<ENC, NMAT, MODE, 7>(a, lds, expert, rb, nt); break;
+    case 8: run_item<ENC, NMAT, MODE, 8>(a, lds, expert, rb, nt); break;
+    default: run_item<ENC, NMAT, MODE, kMaxTT>(a, lds, expert, rb, nt); break;
+  }
+}
+
+namespace {
+
+template <int ENC, int NMAT, int MODE>
+hipError_t launch_cfg(const MfmaArgs& args, hipStream_t stream) {
+  MfmaArgs a = args;
+  const int64_t block_rows = NMAT == 2 ? 64 : 128;
+  a.row_blocks = static_cast<int32_t>((a.rows + block_rows - 1) / block_rows);
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_mfma_kernel<ENC, NMAT, MODE>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+  if (e != hipSuccess) return e;
+  const int64_t items = static_cast<int64_t>(a.row_blocks) * a.tile_bound;
+  const int64_t grid = (items + 7) / 8 * 8;  // every XCD's range rounded up
+  if (grid > 0x7FFFFFFF) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((prefill_mfma_kernel<ENC, NMAT, MODE>), dim3(static_cast<unsigned>(grid)), dim3(kThreads),
+                     kLdsBytes, stream, a);
+  return hipGetLastError();
+}
+
+template <int ENC>
+hipError_t launch_enc(int nmat, int mode, const MfmaArgs& a, hipStream_t stream) {
+  if (nmat == 2 && mode == kModeSilu) return launch_cfg<ENC, 2, kModeSilu>(a, stream);
+  if (nmat == 1 && mode == kModeF32) return launch_cfg<ENC, 1, kModeF32>(a, stream);
+  if (nmat == 1 && mode == kModeBF16) return launch_cfg<ENC, 1, kModeBF16>(a, stream);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+bool prefill_supported(int enc, int64_t rows, int64_t K, int64_t group, int64_t x_rows, int64_t ldx) {
+  if (rows <= 0 || rows % 16 != 0 || K < 256 || K % 128 != 0) return false;
+  // 32-bit byte offsets within one expert's matrix and within the activations
+  if (rows * K * 2 >= (int64_t{1} << 31) || x_rows * ldx * 2 >= (int64_t{1} << 32)) return false;
+  return enc == kBF16 || (group > 0 && group % 128 == 0 && K % group == 0);
+}
+
+hipError_t launch_prefill_mfma(int enc, int nmat, int mode, const MfmaArgs& args, hipStream_t stream) {
+  MfmaArgs a = args;
+  if (!prefill_supported(enc, a.rows, a.K, a.group, 0, a.ldx)) return hipErrorInvalidValue;
+  if (a.tile_bound <= 0) return hipSuccess;
+  if (enc != kBF16) a.scales_per_expert = a.rows * a.K / a.group;
+  if (enc == kQ4) return launch_enc<kQ4>(nmat, mode, a, stream);
+  if (enc == kQ8) return launch_enc<kQ8>(nmat, mode, a, stream);
+  return launch_enc<kBF16>(nmat, mode, a, stream);
+}
+
+}  // namespace uqm

@@ -13,6 +13,8 @@
 // workgroup per 1024 or more routes beyond).
 #include "uqm_route.h"
 
+#include "uqm_prefill.h"
+
 namespace uqm {
 
 // Logit of column e: the bf16 value itself, or the bf16 rounding of the sum of
@@ -200,7 +202,8 @@ __device__ void expert_tables(const int* cnt, int* start, int lane, int E, int32
   }
   int pre = incl - local;
   if (tile_tokens > 0) {
-    // Route tiles: ceil(count / tile_tokens) per expert, in ascending expert id.
+    // Route tiles: ceil(count / tile_tokens) per expert, in ascending expert id
+    // (of equal size where the large-tile kernel takes them).
     int nt4[4];
     int tl = 0;
 #pragma unroll
@@ -218,9 +221,10 @@ __device__ void expert_tables(const int* cnt, int* start, int lane, int E, int32
     int first = pre;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
+      const int step = tile_tokens == kPrefillTileTokens ? route_tile_step(c4[i], tile_tokens) : tile_tokens;
       for (int j = 0; j < nt4[i]; ++j, ++tpos) {
         tiles[2 * tpos] = 4 * lane + i;
-        tiles[2 * tpos + 1] = first + j * tile_tokens;
+        tiles[2 * tpos + 1] = first + j * step;
       }
       first += c4[i];
     }
