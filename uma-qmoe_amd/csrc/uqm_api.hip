@@ -237,15 +237,23 @@ bool routed_uses_stream(const uqm_expert_weights* w) {
 }
 
 // Whether the routed projections of T tokens take the large-tile kernel
-// (uqm_prefill.hip): from 44 routes per active expert on average for Q4 and
-// from 30 for Q8 and BF16. Its items dequantise a row once for up to 144
-// routes; the smaller tiles of uqm_mfma.hip waste less below. Measured, large
-// tiles against small (us per call): Q4 Qwen block 204 vs 200 at 43 routes and
-// 242 vs 306 at 68, Q4 128 experts Zipf 169 vs 173 at 44; Q8 Qwen block 218 vs
-// 231 at 32, 214 vs 206 at 29; BF16 285 vs 300 at 32, 283 vs 282 at 29.
-bool routed_uses_prefill(const uqm_expert_weights* w, int64_t T, int64_t R, double mean) {
+// (uqm_prefill.hip), from the mean routes per active expert: 25 for Q4 (40 with
+// a shared expert beside them), 22 for Q8, 4 for BF16. Its items convert a row
+// once for up to 144 routes and pad to 16; below, the conversion of a 32-row
+// wave outweighs its few MFMAs and the smaller tiles of uqm_mfma.hip are better
+// (BF16 converts nothing). Measured, large tiles against small (us per call;
+// Qwen shapes: whole block with its shared expert, OLMoE: whole block, Zipf: 128
+// experts, routed only):
+//   Q4   Qwen 34 routes 168 vs 160, 43 190 vs 216, 68 215 vs 306;
+//        OLMoE 20 96 vs 89, 25 99 vs 108; Zipf 20 119 vs 117, 25 123 vs 130
+//   Q8   Qwen 17 178 vs 175, 26 193 vs 195, 32 202 vs 233; Zipf 25 146 vs 182
+//   BF16 Qwen 5 231 vs 236, 20 256 vs 253, 32 276 vs 302; Zipf 4 114 vs 118,
+//        12 158 vs 194; OLMoE 4 169 vs 181
+bool routed_uses_prefill(const uqm_expert_weights* w, bool shared, int64_t T, int64_t R, double mean) {
   const int64_t min_t = g_opt_mfma_min_tokens.load(std::memory_order_relaxed);
-  if (min_t <= 0 || T < min_t || mean < (w->encoding == UQM_Q4 ? 44.0 : 30.0)) return false;
+  if (min_t <= 0 || T < min_t) return false;
+  const double least = w->encoding == UQM_Q4 ? (shared ? 40.0 : 25.0) : w->encoding == UQM_Q8 ? 22.0 : 4.0;
+  if (mean < least) return false;
   const int64_t H = w->hidden_size, I = w->intermediate_size;
   return uqm::prefill_supported(w->encoding, I, H, w->group_size, T, H) &&
          uqm::prefill_supported(w->encoding, H, I, w->group_size, R, I);
@@ -255,12 +263,12 @@ bool routed_uses_prefill(const uqm_expert_weights* w, int64_t T, int64_t R, doub
 // per expert on average, 32-route tiles: measured faster than 16 (c5: 80 vs
 // 105 us) and than 64 (c4: 247 vs 271 us), whose 4-wave items take longer per
 // weight byte.
-int routed_tile_tokens(const uqm_expert_weights* w, int64_t T, int64_t k) {
+int routed_tile_tokens(const uqm_expert_weights* w, bool shared, int64_t T, int64_t k) {
   const int64_t R = T * k;
   const int64_t active = R < w->num_experts ? R : w->num_experts;
   const double mean = static_cast<double>(R) / static_cast<double>(active);
   if (routed_uses_stream(w) && R <= g_opt_stream_max_routes.load(std::memory_order_relaxed)) return 0;
-  if (routed_uses_prefill(w, T, R, mean)) return uqm::kPrefillTileTokens;
+  if (routed_uses_prefill(w, shared, T, R, mean)) return uqm::kPrefillTileTokens;
   if (!routed_uses_mfma(w, T)) return 0;
   // 48-route tiles when most experts would otherwise take a second, nearly
   // empty 32-route tile (every tile costs a full pass over the expert's rows)
@@ -471,8 +479,7 @@ int run_routed(const uqm_expert_weights* w, const uint16_t* hidden, int64_t T, i
     d.ldo = H;
     d.part_stride = R * H;
     d.order = kOrderRowFastest;
-    if (prefill)
-      return hip_check(launch_prefill_mfma(w->encoding, 1, kModeF32, d, stream), "down MFMA launch");
+    if (prefill) return hip_check(launch_prefill_mfma(w->encoding, 1, kModeF32, d, stream), "down MFMA launch");
     const MfmaPlan pd = plan_mfma(w->encoding, 1, H, I, nb, active, cus, T > 1 ? kMaxSplit : 1);
     d.ksplit = pd.ksplit;
     *parts = pd.ksplit;
@@ -823,7 +830,7 @@ int uqm_moe_forward(const uqm_expert_weights* weights, const void* hidden, int64
                  at<int32_t>(workspace, L.expert_offsets), at<int32_t>(workspace, L.active_experts),
                  at<int32_t>(workspace, L.counters), at<int32_t>(workspace, L.tiles),
                  at<int32_t>(workspace, L.counters) + 1};
-  const int tile_tokens = routed_tile_tokens(weights, tokens, top_k);
+  const int tile_tokens = routed_tile_tokens(weights, false, tokens, top_k);
   if ((rc = hip_check(launch_route_permute(nullptr, expert_indices, tokens * top_k, weights->num_experts, rt, nullptr,
                                            nullptr, tile_tokens, s),
                       "permute launch")))
@@ -977,7 +984,7 @@ int moe_layer_impl(const uqm_layer_weights* layer, const void* hidden, int64_t t
                  at<int32_t>(workspace, L.counters), at<int32_t>(workspace, L.tiles),
                  at<int32_t>(workspace, L.counters) + 1};
   // top-k and the permutation in one launch when the routes fit one workgroup
-  const int tile_tokens = routed_tile_tokens(w, tokens, k);
+  const int tile_tokens = routed_tile_tokens(w, layer->has_shared != 0, tokens, k);
   const bool fuse_permute = route_topk_permute_fits(tokens, k);
   uint32_t* permute_counter = at<uint32_t>(workspace, L.fused_sync) + kSyncPermuteDone;
   if (router_uses_mfma(H, tokens)) {

@@ -29,13 +29,20 @@
 //   * one work item per workgroup and two workgroups per CU (72 KB of ring, at
 //     most 256 VGPRs): the hardware dispatcher balances items of different
 //     sizes, and one workgroup's start and end run under the other's MFMAs.
-// What bounds it: MFMA and VALU time, which add up on a SIMD (counters at the
-// first size below: 37% and 40% of the cycles, 20% of the wave time waiting).
-// Measured (kernel trace, us, large tiles against uqm_mfma.hip's 32 routes):
-// OLMoE shapes, 4095 tokens (512 routes per expert), Q4: gate/up 325 vs 859,
-// down 214 vs 458; Qwen shapes, routed experts alone: Q4 2048 tokens 168 + 92
-// (233 + 141 beside the shared expert), Q8 999 tokens 137 + 69 (215 + 102),
-// BF16 1535 tokens 203 + 101 (344 + 169; 3.4 TB/s of weights).
+// What bounds it (OLMoE shapes, 4095 tokens): without its loads the loop runs
+// at ~1.5 PFLOP/s, the rate of a large library product on this card; the
+// activation loads into LDS cost 17% of the call, the output writes (268 MB of
+// FP32 rows for the down projection) 14%. BF16 is bound by its weights' 64-byte
+// row segments: 3.8 TB/s.
+// Measured (kernel trace, us, against uqm_mfma.hip's 32 routes): OLMoE shapes,
+// 4095 tokens (512 routes per expert), Q4: gate/up 324 vs 859, down 214 vs 458;
+// Qwen shapes, Q4 2048 tokens 155 + 93 (233 + 141 beside the shared expert),
+// BF16 1535 tokens 183 + 96 (344 + 169).
+// Loads that are not taken by four neighbouring lanes from one 64-byte segment
+// cost 64 cache accesses instead of 16, and weight loads ahead of a stage's
+// made the wait for that stage wait for HBM; with both as they are now the
+// routed experts alone take (us per call, same box) BF16 1535 tokens 280 vs
+// 301, Q8 999 185 vs 196 and 600 163 vs 183, Q4 1000 153 vs 159.
 //
 // MFMA operand layout (v_mfma_f32_16x16x32_bf16): A lane l holds row l%16 and
 // K-slice 8*(l/16)..+7; B lane l holds token l%16, same K-slice; D lane l
@@ -57,15 +64,27 @@ constexpr int kRowBytes = 256;                  // one staged activation row: 12
 constexpr int kTileBytes = 16 * kRowBytes;      // 16 routes of one stage
 constexpr int kMaxTT = kPrefillTileTokens / 16;  // 16-route tiles per item
 constexpr int kRingTiles = 18;                  // 72 KB
-constexpr int kMaxStages = 4;
+constexpr int kMaxStages = 6;
 
 // Stages of the ring for items of TT tiles: small items run through a stage
 // in well under a microsecond and need more of them in flight.
-constexpr int stages_for(int tt) { return kRingTiles / tt < kMaxStages ? kRingTiles / tt : kMaxStages; }
+constexpr int stages_for(int enc, int tt) {
+  const int most = enc == kQ4 ? kMaxStages : 4;
+  return kRingTiles / tt < most ? kRingTiles / tt : most;
+}
+// Weight groups in registers (in flight, or being converted), as many as the
+// tile leaves registers for.
+constexpr int raw_sets_for(int enc, int tt) { return enc == kQ4 && tt <= 6 ? 4 : 2; }
 
-constexpr int kScaleOff = kRingTiles * kTileBytes;             // [stage][128] floats
-constexpr int kRouteOff = kScaleOff + kMaxStages * 128 * 4;    // [kPrefillTileTokens] route ids
-constexpr int kSourceOff = kRouteOff + kPrefillTileTokens * 4;  // [kPrefillTileTokens] activation rows
+// LDS of one workgroup: ring of stages (activations, then the scales: 64
+// floats per wave and stage), route ids, activation rows.
+constexpr int kScaleBytes = 1024;  // per stage
+constexpr int ring_bytes(int enc, int tt) { return stages_for(enc, tt) * (tt * kTileBytes + kScaleBytes); }
+constexpr int max_ring_bytes(int tt) {
+  return tt == 0 ? 0 : (ring_bytes(kQ4, tt) > max_ring_bytes(tt - 1) ? ring_bytes(kQ4, tt) : max_ring_bytes(tt - 1));
+}
+constexpr int kRouteOff = max_ring_bytes(kMaxTT);
+constexpr int kSourceOff = kRouteOff + kPrefillTileTokens * 4;
 constexpr int kLdsBytes = kSourceOff + kPrefillTileTokens * 4;
 static_assert(2 * kLdsBytes <= 160 * 1024, "two workgroups per CU");
 
@@ -118,12 +137,28 @@ __device__ __forceinline__ uint32_t weight_pair(const uint4 (&v)[PEnc<ENC>::kLoa
 }
 
 // 16-byte slot (8 elements, within a group) of the B operand of K-step S for
-// lane quadrant q, matching weight_frag's order.
+// lane quadrant q, matching weight_pair's order.
 template <int ENC>
 __device__ __forceinline__ int x_slot(int q, int S) {
   if constexpr (ENC == kQ4) return 4 * q + S;
   else if constexpr (ENC == kQ8) return 8 * (S >> 1) + 2 * q + (S & 1);
   else return 4 * S + q;
+}
+
+// LDS position of slot s of staged row r is s ^ row_swizzle(r). The LDS serves
+// a 16-byte read of 64 lanes in four turns of 16; each turn holds 16 different
+// rows of a tile, rows 0-3 and 12-15 from one lane quadrant and rows 4-11 from
+// the next one (or the other way round), so their positions are distinct when
+// {swizzle(rows 0-3, 12-15)} and {swizzle(rows 4-11) ^ (slot step from one
+// quadrant to the next)} are: with the row itself for steps of 1 and 2 (BF16,
+// Q8), with bit 2 of the row taken from bit 3 for steps of 4 (Q4). (No bank
+// conflicts in the counters.) An aligned group of four positions holds an
+// aligned group of four slots, so that the four neighbouring lanes which the
+// address unit takes together load 64 contiguous bytes: 16 cache accesses per
+// load of 64 lanes, against 64 when the slots of a group are stored apart.
+template <int ENC>
+__device__ __forceinline__ int row_swizzle(int r) {
+  return ENC == kQ4 ? ((r & 11) | ((r >> 1) & 4)) : (r & 15);
 }
 
 // g / (1 + exp(-g)): the reciprocal refined by one Newton step, as accurate as
@@ -168,10 +203,12 @@ __device__ __forceinline__ void run_item(const MfmaArgs& a, unsigned char* lds, 
   using E = PEnc<ENC>;
   constexpr bool kScaled = ENC != kBF16;
   constexpr int L = E::kLoads;
-  constexpr int D = stages_for(TT);
-  constexpr int kStageBytes = TT * kTileBytes;
+  constexpr int D = stages_for(ENC, TT);
+  constexpr int NR = raw_sets_for(ENC, TT);
+  constexpr int kStageBytes = TT * kTileBytes + kScaleBytes;
   constexpr int kPerStage = TT + (kScaled ? 1 : 0);  // loads into LDS per wave and stage
-  static_assert((D - 2) * kPerStage <= 63, "outstanding loads must fit vmcnt");
+  static_assert((D - 2) * kPerStage + (D - 1) * 2 * L <= 63, "outstanding loads must fit vmcnt");
+  static_assert(NR + 1 >= D - 1, "wait_next counts one weight group per stage from the first stage on");
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -188,17 +225,19 @@ __device__ __forceinline__ void run_item(const MfmaArgs& a, unsigned char* lds, 
   uint32_t woff[2];
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt) {
-    int row = NMAT == 2 ? rb * 64 + 16 * wave + t16 : rb * 128 + 32 * wave + 16 * mt + t16;
+    // a load takes 64 bytes of 16 rows, four neighbouring lanes one row's (16
+    // cache accesses; with the MFMA's own order, 16 rows in neighbouring lanes,
+    // 64); to_operand then moves lane 4 r + c's bytes to lane r + 16 c
+    int row = (lane >> 2) + (NMAT == 2 ? rb * 64 + 16 * wave : rb * 128 + 32 * wave + 16 * mt);
     row = min(row, rows - 1);  // padding rows of the last block repeat the last row
     wbase[mt] = a.w[NMAT == 2 ? mt : 0] + static_cast<int64_t>(expert) * rows * row_bytes;
-    woff[mt] = static_cast<uint32_t>(row) * row_bytes + 16 * q;
+    woff[mt] = static_cast<uint32_t>(row) * row_bytes + 16 * (lane & 3);
   }
   uint32_t xoff[TT];
 #pragma unroll
   for (int j = 0; j < TT; ++j) {
     const int r = 16 * j + 4 * wave + q;  // staged row this lane fills, at position t16
-    const int u = t16 ^ (r & 15);
-    xoff[j] = static_cast<uint32_t>(srcs[r]) * static_cast<uint32_t>(a.ldx * 2) + 16 * x_slot<ENC>(u & 3, u >> 2);
+    xoff[j] = static_cast<uint32_t>(srcs[r]) * static_cast<uint32_t>(a.ldx * 2) + 16 * (t16 ^ row_swizzle<ENC>(r & 15));
   }
   const uint8_t* const x = reinterpret_cast<const uint8_t*>(a.x);
   const float* ssrc = nullptr;
@@ -206,9 +245,12 @@ __device__ __forceinline__ void run_item(const MfmaArgs& a, unsigned char* lds, 
   if constexpr (kScaled) {
     const int G = static_cast<int>(a.K / a.group);
     gdiv = static_cast<int>(a.group / 128);
-    int row = NMAT == 2 ? rb * 64 + lane : rb * 128 + 64 * (wave & 1) + lane;
+    // lanes 0-31: this wave's rows (16 of each matrix, or 32); the others
+    // repeat lane 0's (one more cache access each 16)
+    const int l = lane < 32 ? lane : 0;
+    int row = NMAT == 2 ? rb * 64 + 16 * wave + (l & 15) : rb * 128 + 32 * wave + l;
     row = min(row, rows - 1);
-    ssrc = a.s[NMAT == 2 ? wave & 1 : 0] + static_cast<int64_t>(expert) * a.scales_per_expert +
+    ssrc = a.s[NMAT == 2 ? l >> 4 : 0] + static_cast<int64_t>(expert) * a.scales_per_expert +
            static_cast<int64_t>(row) * G;
   }
 
@@ -221,11 +263,8 @@ __device__ __forceinline__ void run_item(const MfmaArgs& a, unsigned char* lds, 
       asm("" : "+v"(o));  // (extended to 64 bits by the load itself, not kept extended)
       dma16(xg + o, buf + (16 * j + 4 * wave) * kRowBytes);
     }
-    if constexpr (kScaled) {
-      // waves 2 and 3 repeat what waves 0 and 1 load, so that every wave waits
-      // for the same number of loads
-      dma4(ssrc + g / gdiv, __builtin_amdgcn_readfirstlane(lds_base + kScaleOff + slot * 512 + (wave & 1) * 256));
-    }
+    if constexpr (kScaled)
+      dma4(ssrc + g / gdiv, __builtin_amdgcn_readfirstlane(buf + TT * kTileBytes + wave * 256));
   };
   auto load_weights = [&](int g, uint4 (&v)[2][L]) {
 #pragma unroll
@@ -240,44 +279,76 @@ __device__ __forceinline__ void run_item(const MfmaArgs& a, unsigned char* lds, 
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) acc[mt][tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
+  // bytes of lane 4 (lane % 16) + lane / 16
+  const int from = 4 * (4 * t16 + q);
+  auto to_operand = [&](uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from, static_cast<int>(v)));
+  };
+
   uint32_t xo[4];  // LDS byte (within a 16-route tile) of this lane's B operand of each K-step
 #pragma unroll
-  for (int s = 0; s < 4; ++s) xo[s] = static_cast<uint32_t>(t16 * kRowBytes + (((q + 4 * s) ^ t16) << 4));
-  const int srow = NMAT == 2 ? 16 * wave + 4 * q : 32 * wave + 4 * q;
+  for (int s = 0; s < 4; ++s) xo[s] = static_cast<uint32_t>(t16 * kRowBytes + ((x_slot<ENC>(q, s) ^ row_swizzle<ENC>(t16)) << 4));
 
-  // Waits until the next stage is resident: of this wave's loads into LDS only
-  // those of the D - 2 stages after it may be in flight. (Loads complete in
-  // issue order; weight loads in between only make the wait stricter.)
-  auto wait_next = [&]() { wait_loads<(D - 2) * kPerStage>(); };
+  // Waits until the next stage is resident. Loads complete in issue order, and
+  // after that stage's, its body's weight group and the loads of the D - 2
+  // stages behind it with a weight group each were issued: those may be in
+  // flight. Past the main loop the compiler may drop weight loads that nothing
+  // uses, so only the loads into LDS are counted there.
+  auto wait_next = [&](auto exact) {
+    wait_loads<(D - 2) * kPerStage + (decltype(exact)::value ? (D - 1) * 2 * L : 0)>();
+  };
 
   struct Weights {
-    u32x4_t f[2][4];  // A operands of a group: [16-row tile][K-step] (Q4, Q8)
+    u32x4_t f[2][4];  // A operands of a group: [16-row tile][K-step]
   };
   struct Raw {
     uint4 v[2][L];
   };
+  // Q4, Q8: the bytes in the operand's lane order
+  auto reorder = [&](Raw& r) {
+    if constexpr (kScaled) {
+#pragma unroll
+      for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int u = 0; u < L; ++u) {
+          uint4& v = r.v[mt][u];
+          v = make_uint4(to_operand(v.x), to_operand(v.y), to_operand(v.z), to_operand(v.w));
+        }
+    }
+  };
   auto convert = [&](const Raw& r, Weights& w, int unit) {  // pair `unit` (0..31) of a group's operands
     const int mt = unit & 1, S_ = unit >> 3, i = (unit >> 1) & 3;
-    w.f[mt][S_][i] = weight_pair<ENC>(r.v[mt], S_, i);
+    if constexpr (kScaled)
+      w.f[mt][S_][i] = weight_pair<ENC>(r.v[mt], S_, i);
+    else
+      w.f[mt][S_][i] = to_operand(dword_of(r.v[mt][S_], i));
   };
   int slot = 0;
-  // One group (stage). Q4, Q8: its MFMAs from `w`, while `r` (the next group's
-  // bytes) becomes `wn` and the bytes of the group after it are loaded into
-  // `rn`. BF16: its MFMAs from `r`, while the next group's are loaded into `rn`.
-  auto group = [&](int g, const Weights& w, const Raw& r, Weights& wn, Raw& rn) {
-    load_weights(min(g + (kScaled ? 2 : 1), S - 1), rn.v);
-    __builtin_amdgcn_sched_barrier(0);
+  Weights w[2];
+  Raw raw[NR];
+  // Group g (a stage), u = g mod NR: its MFMAs from w[u % 2], while the next
+  // group's bytes are converted into the other one and those of group g + NR
+  // are loaded.
+  auto group = [&](int g, auto u_tag, auto exact) {
+    constexpr int U_ = decltype(u_tag)::value;
+    const Weights& wc = w[U_ & 1];
+    Weights& wn = w[(U_ + 1) & 1];
+    Raw& r = raw[(U_ + 1) % NR];
     // (past the last stage the last one is loaded again, into a buffer nothing
     // reads: a branch here would split the group's code and let the compiler
     // move its arithmetic out of it)
     issue(min(g + D - 1, S - 1), slot == 0 ? D - 1 : slot - 1);
     __builtin_amdgcn_sched_barrier(0);
+    // (behind the stage's loads, so that the wait for that stage does not
+    // include these, which come from HBM)
+    load_weights(min(g + NR, S - 1), raw[U_ % NR].v);
+    __builtin_amdgcn_sched_barrier(0);
     const unsigned char* buf = lds + slot * kStageBytes;
     f32x4_t sc[2];
     if constexpr (kScaled) {
-      const float* sl = reinterpret_cast<const float*>(lds + kScaleOff + slot * 512) + srow;
+      const float* sl = reinterpret_cast<const float*>(buf + TT * kTileBytes + wave * 256) + 4 * q;
 #pragma unroll
-      for (int mt = 0; mt < 2; ++mt) sc[mt] = *reinterpret_cast<const f32x4_t*>(sl + (NMAT == 2 ? 64 : 16) * mt);
+      for (int mt = 0; mt < 2; ++mt) sc[mt] = *reinterpret_cast<const f32x4_t*>(sl + 16 * mt);
     }
     bf16x8_t b[2][4];
     f32x4_t d[2][2];
@@ -292,6 +363,7 @@ __device__ __forceinline__ void run_item(const MfmaArgs& a, unsigned char* lds, 
         for (int e = 0; e < 4; ++e) acc[mt][tt][e] = fmaf(sc[mt][e], d[tt & 1][mt][e], acc[mt][tt][e]);
     };
     read(0);
+    reorder(r);
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
       if (tt + 1 < TT) read(tt + 1);
@@ -304,47 +376,49 @@ __device__ __forceinline__ void run_item(const MfmaArgs& a, unsigned char* lds, 
 #pragma unroll
         for (int mt = 0; mt < 2; ++mt) {
           f32x4_t& c = kScaled ? d[tt & 1][mt] : acc[mt][tt];
-          bf16x8_t af;
-          if constexpr (kScaled)
-            af = __builtin_bit_cast(bf16x8_t, w.f[mt][s]);
-          else
-            af = __builtin_bit_cast(bf16x8_t, r.v[mt][s]);
-          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, b[tt & 1][s], c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wc.f[mt][s]), b[tt & 1][s], c, 0, 0, 0);
         }
       if constexpr (kScaled) {
         if (tt > 0) fold(tt - 1);
-#pragma unroll
-        for (int unit = 32 * tt / TT; unit < 32 * (tt + 1) / TT; ++unit) convert(r, wn, unit);
       }
+#pragma unroll
+      for (int unit = 32 * tt / TT; unit < 32 * (tt + 1) / TT; ++unit) convert(r, wn, unit);
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (kScaled) fold(TT - 1);
-    wait_next();
+    wait_next(exact);
     stage_barrier();  // stage g consumed, stage g + 1 resident
     slot = slot + 1 == D ? 0 : slot + 1;
   };
 
-  Weights w0, w1;
-  Raw r0, r1;
 #pragma unroll
   for (int g = 0; g < D - 1; ++g) issue(min(g, S - 1), g);
   __builtin_amdgcn_sched_barrier(0);
-  load_weights(0, r0.v);
-  if constexpr (kScaled) {
-    load_weights(min(1, S - 1), r1.v);
 #pragma unroll
-    for (int unit = 0; unit < 32; ++unit) convert(r0, w0, unit);
-  }
-  wait_next();
+  for (int g = 0; g < NR; ++g) load_weights(min(g, S - 1), raw[g].v);
+  reorder(raw[0]);
+#pragma unroll
+  for (int unit = 0; unit < 32; ++unit) convert(raw[0], w[0], unit);
+  wait_next(std::false_type{});
   stage_barrier();
-  Raw& ra = kScaled ? r1 : r0;
-  Raw& rz = kScaled ? r0 : r1;
+  constexpr int U = NR;
+  static_assert(NR % 2 == 0, "w alternates");
+  constexpr std::true_type in_loop{};
+  constexpr std::false_type last{};
   int g = 0;
-  for (; g + 1 < S; g += 2) {
-    group(g, w0, ra, w1, rz);
-    group(g + 1, w1, rz, w0, ra);
+  for (; g + U <= S; g += U) {
+    group(g, std::integral_constant<int, 0>{}, in_loop);
+    group(g + 1, std::integral_constant<int, 1>{}, in_loop);
+    if constexpr (U > 2) {
+      group(g + 2, std::integral_constant<int, 2>{}, in_loop);
+      group(g + 3, std::integral_constant<int, 3>{}, in_loop);
+    }
   }
-  if (g < S) group(g, w0, ra, w1, rz);
+  if (g < S) group(g, std::integral_constant<int, 0>{}, last);
+  if constexpr (U > 2) {
+    if (g + 1 < S) group(g + 1, std::integral_constant<int, 1>{}, last);
+    if (g + 2 < S) group(g + 2, std::integral_constant<int, 2>{}, last);
+  }
   wait_loads<0>();  // no load into LDS outlives the workgroup
 
   // ---- outputs ----
@@ -405,7 +479,7 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_mfma_kernel(MfmaArgs a) {
     const int end = __builtin_amdgcn_readfirstlane(a.expert_offsets[expert + 1]);
     nt = min(route_tile_step(end - beg, kPrefillTileTokens), end - first);
   } else {
-    const int step = route_tile_step(a.n_routes, kPrefillTileTokens);
+    const int step = even_step(a.n_routes, a.tile_bound);
     first = tile * step;
     nt = min(step, a.n_routes - first);
   }
