@@ -12,7 +12,9 @@ from dataclasses import replace
 import pytest
 import torch
 
+from oracle import codec as oc
 from oracle import moe as om
+from test_gpu_kernels import assert_bf16_rounded
 from test_gpu_mfma import DEV, close, mfma_on, note, to_dev  # noqa: F401
 from uma_qmoe_amd import synthetic as syn
 
@@ -110,3 +112,28 @@ def test_block_replays_from_a_graph(mfma_on):  # noqa: F811
         torch.cuda.synchronize()
         assert torch.equal(res, ref)
         ext.moe_layer(layer, dense, x, shape.top_k, workspace=ws)
+
+
+# rows: the first that takes the tiles, both sides of one 16-row tile, of the
+# largest tile, several tiles; out features: not a multiple of the 128-row block
+# (16, 1424), below it (64), and one the tiles do not take (1420)
+@pytest.mark.parametrize("encoding", ["q4_group128", "q8_group128", "bf16_le"])
+@pytest.mark.parametrize("rows,n,k", [(25, 1424, 256), (33, 16, 640), (144, 64, 2048), (145, 1424, 384),
+                                      (700, 1420, 256), (1000, 1424, 512)])
+def test_linear_many_rows(hip_ext, encoding, rows, n, k):
+    note(f"linear {encoding} rows={rows} n={n} k={k}")
+    g = torch.Generator().manual_seed(rows + n + k)
+    w = torch.randn(1, n, k, generator=g) * 0.02
+    data, scales = syn.encode_projection(w, encoding)
+    x = torch.randn(rows, k, generator=g).to(torch.bfloat16)
+    xd, wd = x.to(DEV), data[0].to(DEV)
+    if encoding == "q4_group128":
+        deq = oc.q4_dequantize(data.numpy().tobytes(), scales.numpy().tobytes(), (n, k))
+        got = hip_ext.q4_linear(xd, wd, scales[0].to(DEV), n, k, 128)
+    elif encoding == "q8_group128":
+        deq = oc.q8_dequantize(data.numpy().tobytes(), scales.numpy().tobytes(), (n, k))
+        got = hip_ext.q8_linear(xd, wd, scales[0].to(DEV), n, k, 128)
+    else:
+        deq = data[0].float().numpy()
+        got = hip_ext.bf16_linear(xd, wd)
+    assert_bf16_rounded(got, x.float() @ torch.from_numpy(deq).T, "linear")

@@ -688,6 +688,36 @@ static int linear_impl(int enc, const void* input, int64_t rows, const void* w, 
   a.n_routes = static_cast<int32_t>(rows);
   a.out = output;
   a.ldo = out_features;
+  // Many rows: MFMA tiles (uqm_prefill.hip), from 17 rows on for Q8, 25 for Q4
+  // and BF16. The GEMV reads the matrix again every 4 rows (18 to 25 rows cost it
+  // as much as the tiled kernel, bound by its chain of K / 128 stages, takes for
+  // up to ~300). Measured, us per call, 1408 x 2048: Q4 16 rows 12.2 vs 10.8, 24
+  // 12.1 vs 14.6, 137 12.9 vs 71; Q8 16 13.5 vs 13.8, 137 vs 100; BF16 24 16.0 vs
+  // 17.2, 137 vs 91; 768 x 2048: Q4 20 12.1 vs 10.9, 24 12.2 vs 12.6.
+  if (rows >= (enc == UQM_Q8 ? 17 : 25) && rows <= 0x7FFFFFFF && reinterpret_cast<uintptr_t>(output) % 8 == 0 &&
+      prefill_supported(enc, out_features, in_features, group_size, rows, in_features)) {
+    const int64_t row_blocks = (out_features + 127) / 128;
+    const int64_t fewest = (rows + kPrefillTileTokens - 1) / kPrefillTileTokens;
+    const int64_t most = (rows + 15) / 16;
+    // as many tiles as fill the CUs (each at least 16 rows, at most the kernel's)
+    int64_t tiles = device_cus() / row_blocks;
+    tiles = tiles < fewest ? fewest : (tiles > most ? most : tiles);
+    const int64_t step = even_step(static_cast<int>(rows), static_cast<int>(tiles));
+    MfmaArgs m{};
+    m.w[0] = a.w[0];
+    m.s[0] = s;
+    m.rows = out_features;
+    m.K = in_features;
+    m.group = group_size;
+    m.x = a.x;
+    m.ldx = in_features;
+    m.x_div = 1;
+    m.n_routes = static_cast<int32_t>(rows);
+    m.tile_bound = static_cast<int32_t>((rows + step - 1) / step);
+    m.out = output;
+    m.ldo = out_features;
+    return hip_check(launch_prefill_mfma(enc, 1, kModeBF16, m, static_cast<hipStream_t>(stream)), "linear launch");
+  }
   const int nt = static_cast<int>(rows < 4 ? rows : 4);
   return hip_check(launch_expert_gemv(enc, 1, kModeBF16, a, 1, nt, static_cast<hipStream_t>(stream)), "linear launch");
 }
