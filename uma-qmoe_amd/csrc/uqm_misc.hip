@@ -160,10 +160,63 @@ hipError_t launch_combine(const float* y, int y_parts, int64_t y_stride, const u
   }
 }
 
-__global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* __restrict__ x, int64_t H,
-                                                      const uint16_t* __restrict__ weight, float eps,
-                                                      uint16_t* __restrict__ out) {
-  __shared__ float part[4];
+// One workgroup per row; a thread keeps its elements in registers between the
+// sum and the scaling. VEC: rows of a multiple of 8 elements, at most 8 per
+// thread and pass, 16-byte loads and stores (the row's one round trip through
+// memory is what the launch costs: 1535 rows of 2048 5.1 us against 10.5 with
+// one element at a time and the row read twice, 6 rows 3.6 against 9.2).
+constexpr int kNormThreads = 256;
+constexpr int kNormPasses = 4;  // 16-byte loads per thread: rows up to 8192 elements
+
+__device__ __forceinline__ float block_sum(float v, float* part) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return part[0] + part[1] + part[2] + part[3];
+}
+
+__global__ __launch_bounds__(kNormThreads) void rmsnorm_vec_kernel(const uint16_t* __restrict__ x, int H,
+                                                                   const uint16_t* __restrict__ weight, float eps,
+                                                                   uint16_t* __restrict__ out) {
+  __shared__ float part[kNormThreads / 64];
+  const uint16_t* xr = x + static_cast<int64_t>(blockIdx.x) * H;
+  uint16_t* orow = out + static_cast<int64_t>(blockIdx.x) * H;
+  uint4 v[kNormPasses], w[kNormPasses];
+#pragma unroll
+  for (int p = 0; p < kNormPasses; ++p) {
+    const int i = 8 * (kNormThreads * p + static_cast<int>(threadIdx.x));
+    v[p] = i < H ? ldg16(xr + i) : make_uint4(0u, 0u, 0u, 0u);
+    w[p] = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);  // bf16 ones
+    if (weight != nullptr && i < H) w[p] = ldg16(weight + i);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int p = 0; p < kNormPasses; ++p) {
+    const uint32_t q[4] = {v[p].x, v[p].y, v[p].z, v[p].w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ss = fmaf(bf16hi(q[j]), bf16hi(q[j]), fmaf(bf16lo(q[j]), bf16lo(q[j]), ss));
+  }
+  const float r = rsqrtf(block_sum(ss, part) / static_cast<float>(H) + eps);
+#pragma unroll
+  for (int p = 0; p < kNormPasses; ++p) {
+    const int i = 8 * (kNormThreads * p + static_cast<int>(threadIdx.x));
+    const uint32_t q[4] = {v[p].x, v[p].y, v[p].z, v[p].w};
+    const uint32_t u[4] = {w[p].x, w[p].y, w[p].z, w[p].w};
+    uint32_t o[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t n = pack_bf16x2(bf16lo(q[j]) * r, bf16hi(q[j]) * r);
+      o[j] = pack_bf16x2(bf16lo(u[j]) * bf16lo(n), bf16hi(u[j]) * bf16hi(n));
+    }
+    if (i < H) *reinterpret_cast<uint4*>(orow + i) = make_uint4(o[0], o[1], o[2], o[3]);
+  }
+}
+
+// Any row length and alignment, one element at a time.
+__global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const uint16_t* __restrict__ x, int64_t H,
+                                                               const uint16_t* __restrict__ weight, float eps,
+                                                               uint16_t* __restrict__ out) {
+  __shared__ float part[kNormThreads / 64];
   const uint16_t* xr = x + blockIdx.x * H;
   uint16_t* orow = out + blockIdx.x * H;
   float ss = 0.f;
@@ -171,11 +224,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* __restrict
     const float v = bf16_to_f32(xr[i]);
     ss = fmaf(v, v, ss);
   }
-  ss = wave_sum(ss);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
-  __syncthreads();
-  const float total = part[0] + part[1] + part[2] + part[3];
-  const float r = rsqrtf(total / static_cast<float>(H) + eps);
+  const float r = rsqrtf(block_sum(ss, part) / static_cast<float>(H) + eps);
   for (int64_t i = threadIdx.x; i < H; i += blockDim.x) {
     const float nv = round_bf16(bf16_to_f32(xr[i]) * r);
     const float wv = weight != nullptr ? bf16_to_f32(weight[i]) : 1.0f;
@@ -186,8 +235,14 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* __restrict
 hipError_t launch_rmsnorm(const uint16_t* x, int64_t rows, int64_t H, const uint16_t* weight, float eps,
                           uint16_t* out, hipStream_t stream) {
   if (rows <= 0) return hipSuccess;
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3(static_cast<unsigned>(rows)), dim3(256), 0, stream, x, H, weight, eps,
-                     out);
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out) |
+                         reinterpret_cast<uintptr_t>(weight);  // (NULL weight: ones)
+  if (H % 8 == 0 && H <= 8 * kNormThreads * kNormPasses && (bits & 15u) == 0)
+    hipLaunchKernelGGL(rmsnorm_vec_kernel, dim3(static_cast<unsigned>(rows)), dim3(kNormThreads), 0, stream, x,
+                       static_cast<int>(H), weight, eps, out);
+  else
+    hipLaunchKernelGGL(rmsnorm_kernel, dim3(static_cast<unsigned>(rows)), dim3(kNormThreads), 0, stream, x, H, weight,
+                       eps, out);
   return hipGetLastError();
 }
 
