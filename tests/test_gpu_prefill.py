@@ -15,7 +15,7 @@ import torch
 from oracle import codec as oc
 from oracle import moe as om
 from test_gpu_kernels import assert_bf16_rounded
-from test_gpu_mfma import DEV, close, mfma_on, note, to_dev  # noqa: F401
+from test_gpu_mfma import DEV, RAGGED, close, dense_cpu, layout_of, mfma_on, note, to_dev  # noqa: F401
 from uma_qmoe_amd import synthetic as syn
 
 pytestmark = pytest.mark.gpu
@@ -137,3 +137,24 @@ def test_linear_many_rows(hip_ext, encoding, rows, n, k):
         deq = data[0].float().numpy()
         got = hip_ext.bf16_linear(xd, wd)
     assert_bf16_rounded(got, x.float() @ torch.from_numpy(deq).T, "linear")
+
+
+@pytest.mark.parametrize("which,t", [("ragged", 4300), ("ragged", 9700), ("c2", 2100)])
+def test_dense_256_row_items(mfma_on, which, t):  # noqa: F811
+    """The shared expert on 256 x 256 items. The planner takes them for the
+    ragged shape's gate/up at 4300 tokens (1344 rows: the last 128-row half
+    block half full; 17 token tiles, the last one partial) and for its down
+    projection at 9700 (1088 rows: 64 in the last block), and for both c2
+    projections at 2100 tokens (K split in four)."""
+    shape = RAGGED if which == "ragged" else syn.C2
+    note(f"dense 256 rows {which} t={t}")
+    layer = syn.build_experts(shape, device=DEV)
+    dense = syn.build_dense(shape, device=DEV)
+    x = syn.hidden_states(shape, t, seed=t)
+    out, _logits, weights, indices = mfma_on.moe_layer(layer, dense, x.to(DEV), shape.top_k)
+    pick = torch.randperm(t, generator=torch.Generator().manual_seed(t))[:24]
+    pick = torch.unique(torch.cat([pick, torch.tensor([0, t - 1])]))
+    ref, *_ = om.qwen_block(x[pick], layout_of(shape, dense_cpu(dense)), syn.DeviceLayerReader({0: layer}), 0,
+                            routes=(weights.cpu()[pick], indices.cpu()[pick]))
+    close(out.cpu()[pick], ref, f"dense 256 rows {which} t={t}")
+    assert torch.isfinite(out.float()).all()

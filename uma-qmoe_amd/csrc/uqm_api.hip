@@ -552,9 +552,7 @@ int run_shared(const uqm_layer_weights* layer, const uint16_t* x, int64_t T, int
     g.T = T;
     g.out = at<uint16_t>(ws, L.h_shared);
     g.ldo = Is;
-    g.ksplit = 1;
-    const DensePlan pg = plan_dense(2, Is, H, T, cus, 1);
-    int rc = hip_check(launch_dense_mfma(2, g, pg.waves, cus, stream), "shared gate/up dense launch");
+    int rc = hip_check(launch_dense_mfma(2, g, plan_dense(2, Is, H, T, cus, 1), cus, stream), "shared gate/up dense launch");
     if (rc) return rc;
     DenseArgs d{};
     d.w[0] = static_cast<const uint16_t*>(layer->shared_down);
@@ -567,9 +565,8 @@ int run_shared(const uqm_layer_weights* layer, const uint16_t* x, int64_t T, int
     d.ldo = H;
     d.part_stride = T * H;
     const DensePlan pd = plan_dense(1, H, Is, T, cus, kMaxSplit);
-    d.ksplit = pd.ksplit;
-    *parts = d.ksplit;
-    return hip_check(launch_dense_mfma(1, d, pd.waves, cus, stream), "shared down dense launch");
+    *parts = pd.ksplit;
+    return hip_check(launch_dense_mfma(1, d, pd, cus, stream), "shared down dense launch");
   }
   if (shared_uses_mfma(H, Is, T)) {
     // Up to 32 tokens: 16-token tiles, so that the plan can split K over

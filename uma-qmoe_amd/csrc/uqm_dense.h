@@ -31,16 +31,18 @@ constexpr int64_t kDenseMinTokens = 128;
 
 bool dense_supported(int64_t rows, int64_t K, int64_t T);
 
-// Workgroup size (4 or 8 waves: 128- or 256-token items) and K split (kModeF32
-// only, at most max_split) with the least estimated time on cus CUs.
+// Work item (4 or 8 waves: 128 or 256 tokens; 128 or, with 8 waves, 256 weight
+// rows, both matrices of gate/up together) and K split (kModeF32 only, at most
+// max_split) with the least estimated time on cus CUs.
 struct DensePlan {
   int waves;
+  int rows;
   int ksplit;
 };
 DensePlan plan_dense(int nmat, int64_t rows, int64_t K, int64_t T, int cus, int max_split);
 
 // nmat 2 = gate/up with the SiLU epilogue, 1 = FP32 rows; cus = compute units
 // the persistent grid may take.
-hipError_t launch_dense_mfma(int nmat, const DenseArgs& a, int waves, int cus, hipStream_t stream);
+hipError_t launch_dense_mfma(int nmat, const DenseArgs& a, const DensePlan& plan, int cus, hipStream_t stream);
 
 }  // namespace uqm

@@ -11,12 +11,13 @@
 // then run its MFMAs in lock step. Here the output tile is square:
 //   * a workgroup of 4 or 8 waves computes 128 weight rows x 128 or 256
 //     tokens, each wave a 64 x 64 block: 4 row tiles x 4 token tiles of
-//     v_mfma_f32_16x16x32_bf16 (64 FP32 accumulators per lane). Gate/up items
-//     take rows r .. r+63 of both matrices and give each wave the same 32 rows
-//     of gate and of up, so the SiLU epilogue pairs them in registers;
+//     v_mfma_f32_16x16x32_bf16 (64 FP32 accumulators per lane), or (8 waves)
+//     256 rows x 256 tokens in blocks of 128 x 64. Gate/up items take half of
+//     their rows from each matrix and give each wave the same rows of gate and
+//     of up, so the SiLU epilogue pairs them in registers;
 //   * K advances 64 elements per stage; every wave issues a quarter of each
 //     stage's loads (global_load_lds, 16 bytes per lane, no registers) into a
-//     ring of 4 stages of 32 KB or 3 of 48 KB, all but one ahead of the stage
+//     ring of 4 stages of 32 KB, 3 of 48 KB or 2 of 64 KB, all but one ahead of the stage
 //     being computed;
 //   * each 32-element chunk's fragments are read from LDS while the previous
 //     chunk's MFMAs run (two register sets); the barrier of a stage only hands
@@ -43,18 +44,23 @@ typedef __attribute__((address_space(3))) void dense_lds_t;
 
 constexpr int kStepK = 64;             // K elements per stage
 constexpr int kRowBytes = 2 * kStepK;  // one staged row
-constexpr int kRegionA = 128 * kRowBytes;  // 128 weight rows
-
-// WAVES = 4: 128-token items, a ring of 4 stages of 32 KB (one wave per SIMD);
-// WAVES = 8: 256-token items, 3 stages of 48 KB (two waves per SIMD: twice the
-// MFMA work per stage barrier, and one wave's MFMAs run while the other waits).
-template <int WAVES>
+// Items of ROWS weight rows (both matrices of gate/up together) x 32 WAVES
+// tokens, each wave ROWS / 2 x 64 of them:
+// WAVES = 4, ROWS = 128: a ring of 4 stages of 32 KB (one wave per SIMD);
+// WAVES = 8, ROWS = 128: 3 stages of 48 KB (two waves per SIMD: twice the
+// MFMA work per stage barrier, and one wave's MFMAs run while the other waits);
+// WAVES = 8, ROWS = 256: 2 stages of 64 KB; a wave's 128 x 64 block reads 0.375
+// KB of fragments per MFMA instead of 0.5.
+template <int WAVES, int ROWS>
 struct DenseCfg {
   static_assert(WAVES == 4 || WAVES == 8, "4 or 8 waves");
+  static_assert(ROWS == 128 || (ROWS == 256 && WAVES == 8), "128 rows, or 256 with 8 waves");
+  static constexpr int kRowTiles = ROWS / 32;               // 16-row tiles per wave
   static constexpr int kTokens = 32 * WAVES;                // tokens per work item
+  static constexpr int kRegionA = ROWS * kRowBytes;
   static constexpr int kRegionB = kTokens * kRowBytes;      // the item's tokens
   static constexpr int kStageBytes = kRegionA + kRegionB;
-  static constexpr int kStages = WAVES == 8 ? 3 : 4;
+  static constexpr int kStages = ROWS == 256 ? 2 : (WAVES == 8 ? 3 : 4);
   static constexpr int kLoadsA = kRegionA / 1024 / WAVES;  // 1 KB loads per wave and stage
   static constexpr int kLoadsB = kRegionB / 1024 / WAVES;
   static constexpr int kLoadsPerWave = kLoadsA + kLoadsB;
@@ -122,13 +128,13 @@ __device__ __forceinline__ uint32_t slot_at(int row, int slot) {
 // the accumulators stay in VGPRs with each MFMA's result in its own input
 // registers; with 512 the compiler moves them through AGPRs around every MFMA.
 // One workgroup per CU runs, bound by its LDS ring.)
-template <int MODE, int WAVES>
+template <int MODE, int WAVES, int ROWS>
 __global__ __launch_bounds__(64 * WAVES, 2) void dense_mfma_kernel(DenseArgs a) {
-  using C = DenseCfg<WAVES>;
+  using C = DenseCfg<WAVES, ROWS>;
   constexpr int kTokens = C::kTokens, kStages = C::kStages, kStageBytes = C::kStageBytes;
-  constexpr int kLoadsA = C::kLoadsA, kLoadsB = C::kLoadsB;
+  constexpr int kLoadsA = C::kLoadsA, kLoadsB = C::kLoadsB, kRegionA = C::kRegionA, MT = C::kRowTiles;
   constexpr bool kSilu = MODE == kModeSilu;
-  constexpr int RB = kSilu ? 64 : 128;  // rows per item per matrix
+  constexpr int RB = kSilu ? ROWS / 2 : ROWS;  // rows per item per matrix
   extern __shared__ __align__(16) unsigned char lds[];
 
   const int lane = threadIdx.x & 63;
@@ -170,7 +176,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void dense_mfma_kernel(DenseArgs a) 
   // source rows are set up once per item (clamped to the last row / token).
   // (kernel arguments read once: a scalar load in flight inside the loop would
   // make every LDS wait there a full one)
-  const uint16_t* const wsel = kSilu && wave >= WAVES / 2 ? a.w[1] : a.w[0];  // weight loads 8-15: up rows
+  const uint16_t* const wsel = kSilu && wave >= WAVES / 2 ? a.w[1] : a.w[0];  // the second half of the weight loads: up rows
   const uint16_t* const xbase = a.x;
   const int64_t rows = a.rows, K = a.K, T = a.T, ldx = a.ldx, ldo = a.ldo, part_stride = a.part_stride;
   void* const out = a.out;
@@ -184,7 +190,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void dense_mfma_kernel(DenseArgs a) 
     for (int u = 0; u < kLoadsA; ++u) {
       const int row = 8 * (kLoadsA * wave + u) + (lane >> 3);
       const int slot = (lane & 7) ^ ((row >> 1) & 7);
-      int64_t wrow = static_cast<int64_t>(it.rb) * RB + (kSilu ? (row & 63) : row);
+      int64_t wrow = static_cast<int64_t>(it.rb) * RB + (kSilu ? (row & (RB - 1)) : row);
       if (wrow >= rows) wrow = rows - 1;
       wsrc[u] = wsel + wrow * K + 8 * slot;
     }
@@ -213,26 +219,30 @@ __global__ __launch_bounds__(64 * WAVES, 2) void dense_mfma_kernel(DenseArgs a) 
 
   // ---- fragments of one 32-element chunk ----
   struct Frags {
-    bf16x8_t fa[4];
+    bf16x8_t fa[MT];
     bf16x8_t fb[4];
   };
   // staged row of this lane in A tile mt (its base is a multiple of 16, so the
   // slot swizzle depends on r16 only)
-  auto a_base = [&](int mt) { return kSilu ? 64 * (mt >> 1) + 32 * wr + 16 * (mt & 1) : 64 * wr + 16 * mt; };
+  // (gate/up: half of the wave's tiles gate rows, then the same rows of up)
+  constexpr int HT = MT / 2;
+  auto a_base = [&](int mt) {
+    return kSilu ? RB * (mt / HT) + 16 * HT * wr + 16 * (mt % HT) : 16 * MT * wr + 16 * mt;
+  };
   const uint32_t off0 = slot_at(r16, q), off1 = slot_at(r16, 4 + q);
   auto read = [&](int g, int c, Frags& f) {
     const unsigned char* buf = lds + (g % kStages) * kStageBytes + (c ? off1 : off0);
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) f.fa[mt] = *reinterpret_cast<const bf16x8_t*>(buf + a_base(mt) * kRowBytes);
+    for (int mt = 0; mt < MT; ++mt) f.fa[mt] = *reinterpret_cast<const bf16x8_t*>(buf + a_base(mt) * kRowBytes);
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt)
       f.fb[tt] = *reinterpret_cast<const bf16x8_t*>(buf + kRegionA + (64 * wt + 16 * tt) * kRowBytes);
   };
 
-  f32x4_t acc[4][4];
+  f32x4_t acc[MT][4];
   auto mfma = [&](const Frags& f) {
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt)
         acc[mt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.fa[mt], f.fb[tt], acc[mt][tt], 0, 0, 0);
@@ -246,20 +256,20 @@ __global__ __launch_bounds__(64 * WAVES, 2) void dense_mfma_kernel(DenseArgs a) 
       if (t >= T) continue;
       if constexpr (kSilu) {
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) {
-          const int64_t n = static_cast<int64_t>(it.rb) * RB + 32 * wr + 16 * rt + 4 * q;
+        for (int rt = 0; rt < HT; ++rt) {
+          const int64_t n = static_cast<int64_t>(it.rb) * RB + 16 * HT * wr + 16 * rt + 4 * q;
           if (n >= rows) continue;
           uint16_t h[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) h[e] = f32_to_bf16(silu(round_bf16(acc[rt][tt][e])) * round_bf16(acc[2 + rt][tt][e]));
+          for (int e = 0; e < 4; ++e) h[e] = f32_to_bf16(silu(round_bf16(acc[rt][tt][e])) * round_bf16(acc[HT + rt][tt][e]));
           const uint2 v = make_uint2(static_cast<uint32_t>(h[0]) | (static_cast<uint32_t>(h[1]) << 16),
                                      static_cast<uint32_t>(h[2]) | (static_cast<uint32_t>(h[3]) << 16));
           *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + t * ldo + n) = v;
         }
       } else {
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
-          const int64_t n = static_cast<int64_t>(it.rb) * RB + 64 * wr + 16 * mt + 4 * q;
+        for (int mt = 0; mt < MT; ++mt) {
+          const int64_t n = static_cast<int64_t>(it.rb) * RB + 16 * MT * wr + 16 * mt + 4 * q;
           if (n >= rows) continue;
           float* dst = static_cast<float*>(out) + it.split * part_stride + t * ldo + n;
           *reinterpret_cast<float4*>(dst) = make_float4(acc[mt][tt][0], acc[mt][tt][1], acc[mt][tt][2], acc[mt][tt][3]);
@@ -280,7 +290,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void dense_mfma_kernel(DenseArgs a) 
   read(0, 0, f0);
   for (int i = 0, g = 0; i < nit; ++i) {
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) acc[mt][tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     for (int j = 0; j < S; ++j, ++g) {
@@ -305,25 +315,25 @@ bool dense_supported(int64_t rows, int64_t K, int64_t T) {
 
 namespace {
 
-int64_t dense_items(int nmat, int64_t rows, int64_t T, int waves, int ksplit) {
-  const int64_t rb = nmat == 2 ? 64 : 128;
+int64_t dense_items(int nmat, int64_t rows, int64_t T, int waves, int item_rows, int ksplit) {
+  const int64_t rb = item_rows / nmat;
   const int64_t tok = 32 * waves;
   return (rows + rb - 1) / rb * ksplit * ((T + tok - 1) / tok);
 }
 
-template <int MODE, int WAVES>
+template <int MODE, int WAVES, int ROWS>
 hipError_t launch_cfg(const DenseArgs& a, int cus, hipStream_t stream) {
-  using C = DenseCfg<WAVES>;
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_mfma_kernel<MODE, WAVES>),
+  using C = DenseCfg<WAVES, ROWS>;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_mfma_kernel<MODE, WAVES, ROWS>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(C::kLds));
   if (e != hipSuccess) return e;
   // persistent grid: one workgroup per CU (the ring takes 128-144 KB of LDS),
   // a multiple of 8 so that every XCD gets the same number
-  const int64_t items = dense_items(MODE == kModeSilu ? 2 : 1, a.rows, a.T, WAVES, a.ksplit);
+  const int64_t items = dense_items(MODE == kModeSilu ? 2 : 1, a.rows, a.T, WAVES, ROWS, a.ksplit);
   int64_t grid = cus < items ? cus : items;
   grid = (grid + 7) & ~static_cast<int64_t>(7);
   if (grid < 8) grid = 8;
-  hipLaunchKernelGGL((dense_mfma_kernel<MODE, WAVES>), dim3(static_cast<unsigned>(grid)), dim3(C::kThreads), C::kLds,
+  hipLaunchKernelGGL((dense_mfma_kernel<MODE, WAVES, ROWS>), dim3(static_cast<unsigned>(grid)), dim3(C::kThreads), C::kLds,
                      stream, a);
   return hipGetLastError();
 }
@@ -331,37 +341,52 @@ hipError_t launch_cfg(const DenseArgs& a, int cus, hipStream_t stream) {
 }  // namespace
 
 DensePlan plan_dense(int nmat, int64_t rows, int64_t K, int64_t T, int cus, int max_split) {
-  // Relative time of one stage: the 8-wave item (128 x 256) takes ~1.4 times
-  // as long per stage as the 4-wave one (128 x 128) for twice the work
-  // (c4 gate/up: 1.1 vs 0.79 us per stage).
+  // Relative time of one stage per item size: the 8-wave item (128 x 256) takes
+  // ~1.4 times as long per stage as the 4-wave one (128 x 128) for twice the
+  // work (c4 gate/up: 1.1 vs 0.79 us per stage), the 256 x 256 one ~2 times for
+  // four times (gate/up at 2048 tokens on 192 CUs 129 vs 145 us with 128 x 256).
+  // With 2.0 the block takes (us per call, against no 256-row items) 365 vs 398
+  // at 2048 tokens, 278 vs 286 at 1400, 192 vs 194 at 700; from 2.3 on the
+  // planner leaves 1400 and 1535 tokens on 128 rows (287 vs 278, 397 vs 383).
+  struct Size {
+    int waves, rows;
+    double stage;
+  };
+  const Size sizes[] = {{4, 128, 1.0}, {8, 128, 1.4}, {8, 256, 2.0}};
   const int64_t steps = K / kStepK;
   const int64_t grid = cus < 8 ? 8 : cus;
-  DensePlan best{4, 1};
+  DensePlan best{4, 128, 1};
   double best_cost = -1.0;
-  for (int waves = 4; waves <= 8; waves *= 2) {
+  for (const Size& z : sizes) {
     for (int ks = 1; ks <= (nmat == 2 ? 1 : max_split); ks *= 2) {
       if (steps % ks != 0) continue;
-      const int64_t rounds = (dense_items(nmat, rows, T, waves, ks) + grid - 1) / grid;
-      const double cost = static_cast<double>(rounds * (steps / ks)) * (waves == 8 ? 1.4 : 1.0);
-      if (best_cost < 0.0 || cost < best_cost) {  // ties: fewer waves, smaller split
+      const int64_t rounds = (dense_items(nmat, rows, T, z.waves, z.rows, ks) + grid - 1) / grid;
+      const double cost = static_cast<double>(rounds * (steps / ks)) * z.stage;
+      if (best_cost < 0.0 || cost < best_cost) {  // ties: smaller items, smaller split
         best_cost = cost;
-        best = DensePlan{waves, ks};
+        best = DensePlan{z.waves, z.rows, ks};
       }
     }
   }
   return best;
 }
 
-hipError_t launch_dense_mfma(int nmat, const DenseArgs& args, int waves, int cus, hipStream_t stream) {
+hipError_t launch_dense_mfma(int nmat, const DenseArgs& args, const DensePlan& plan, int cus, hipStream_t stream) {
   DenseArgs a = args;
   if (nmat != 1 && nmat != 2) return hipErrorInvalidValue;
-  if (waves != 4 && waves != 8) return hipErrorInvalidValue;
+  if (plan.waves != 4 && plan.waves != 8) return hipErrorInvalidValue;
+  if (plan.rows != 128 && (plan.rows != 256 || plan.waves != 8)) return hipErrorInvalidValue;
   if (!dense_supported(a.rows, a.K, a.T)) return hipErrorInvalidValue;
-  if (a.ksplit < 1) a.ksplit = 1;
+  a.ksplit = plan.ksplit < 1 ? 1 : plan.ksplit;
   if (nmat == 2 && a.ksplit != 1) return hipErrorInvalidValue;
   if ((a.K / kStepK) % a.ksplit != 0) return hipErrorInvalidValue;
-  if (nmat == 2) return waves == 8 ? launch_cfg<kModeSilu, 8>(a, cus, stream) : launch_cfg<kModeSilu, 4>(a, cus, stream);
-  return waves == 8 ? launch_cfg<kModeF32, 8>(a, cus, stream) : launch_cfg<kModeF32, 4>(a, cus, stream);
+  if (nmat == 2) {
+    if (plan.rows == 256) return launch_cfg<kModeSilu, 8, 256>(a, cus, stream);
+    return plan.waves == 8 ? launch_cfg<kModeSilu, 8, 128>(a, cus, stream)
+                           : launch_cfg<kModeSilu, 4, 128>(a, cus, stream);
+  }
+  if (plan.rows == 256) return launch_cfg<kModeF32, 8, 256>(a, cus, stream);
+  return plan.waves == 8 ? launch_cfg<kModeF32, 8, 128>(a, cus, stream) : launch_cfg<kModeF32, 4, 128>(a, cus, stream);
 }
 
 }  // namespace uqm
