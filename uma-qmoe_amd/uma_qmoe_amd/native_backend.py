@@ -65,7 +65,13 @@ def observed_native_platform(torch: Any, device: Any = 0) -> str:
 
 
 def _stream_handle(torch: Any, device: Any) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    """Handle of the device's current stream. Asked for twice per call, so the
+    raw handle is taken without building a Stream object (0.2 against 2.0 us;
+    an eager one-token block spends about as long on the host as on the GPU)."""
+    index = device.index if isinstance(device, torch.device) else None
+    if index is None:
+        return int(torch.cuda.current_stream(device).cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def _ptr(t: Any) -> int | None:
