@@ -1,5 +1,6 @@
-"""RMSNorm launch against the CPU oracle: vector rows (multiples of 8, up to
-8192), the element-wise form beyond and for unaligned pointers.
+"""RMSNorm launch against the CPU oracle: vector rows (multiples of 8, 128 to
+8192, in one, two or four passes), the element-wise form for the others and for
+unaligned pointers.
 
 The FP32 sum of squares runs in another order than the oracle's (relative error
 below 1e-5 here), so a value can round to the neighbouring bf16 once in the
@@ -17,7 +18,8 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("rows,hidden,offset", [(1, 8, 0), (6, 2048, 0), (3, 2056, 0), (2, 8192, 0), (2, 8200, 0),
-                                                (5, 2047, 0), (3, 2048, 1)])
+                                                (5, 2047, 0), (3, 2048, 1), (4, 120, 0), (4, 128, 0), (3, 136, 0),
+                                                (2, 4096, 0), (2, 4104, 0)])
 @pytest.mark.parametrize("weighted", [False, True])
 def test_rmsnorm_rows(hip_ext, rows, hidden, offset, weighted):
     print(f"[case] rmsnorm {rows}x{hidden}+{offset} weighted={weighted}", flush=True)

@@ -161,12 +161,17 @@ hipError_t launch_combine(const float* y, int y_parts, int64_t y_stride, const u
 }
 
 // One workgroup per row; a thread keeps its elements in registers between the
-// sum and the scaling. VEC: rows of a multiple of 8 elements, at most 8 per
-// thread and pass, 16-byte loads and stores (the row's one round trip through
-// memory is what the launch costs: 1535 rows of 2048 5.1 us against 10.5 with
-// one element at a time and the row read twice, 6 rows 3.6 against 9.2).
+// sum and the scaling. Here rows of a multiple of 8 elements, PASSES 16-byte
+// loads and stores per thread (the row's one round trip through memory is what
+// the launch costs: 1535 rows of 2048 5.1 us against 10.5 with one element at a
+// time and the row read twice, 6 rows 3.6 against 9.2). PASSES is the fewest
+// that cover the row: with four for every row the arithmetic of the empty
+// passes was most of a narrow row's time (16384 rows of 256 8.8 us against 15.4,
+// element-wise 12.8). Rows below 128 elements stay element-wise: a quarter of a
+// wave or less would load them (16384 rows of 64 7.4 us against 8.0; of 128 9.5
+// against 8.3).
 constexpr int kNormThreads = 256;
-constexpr int kNormPasses = 4;  // 16-byte loads per thread: rows up to 8192 elements
+constexpr int kNormPasses = 4;  // most 16-byte loads per thread: rows up to 8192 elements
 
 __device__ __forceinline__ float block_sum(float v, float* part) {
   v = wave_sum(v);
@@ -175,15 +180,16 @@ __device__ __forceinline__ float block_sum(float v, float* part) {
   return part[0] + part[1] + part[2] + part[3];
 }
 
+template <int PASSES>
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_vec_kernel(const uint16_t* __restrict__ x, int H,
                                                                    const uint16_t* __restrict__ weight, float eps,
                                                                    uint16_t* __restrict__ out) {
   __shared__ float part[kNormThreads / 64];
   const uint16_t* xr = x + static_cast<int64_t>(blockIdx.x) * H;
   uint16_t* orow = out + static_cast<int64_t>(blockIdx.x) * H;
-  uint4 v[kNormPasses], w[kNormPasses];
+  uint4 v[PASSES], w[PASSES];
 #pragma unroll
-  for (int p = 0; p < kNormPasses; ++p) {
+  for (int p = 0; p < PASSES; ++p) {
     const int i = 8 * (kNormThreads * p + static_cast<int>(threadIdx.x));
     v[p] = i < H ? ldg16(xr + i) : make_uint4(0u, 0u, 0u, 0u);
     w[p] = make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);  // bf16 ones
@@ -191,14 +197,14 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_vec_kernel(const uint16_
   }
   float ss = 0.f;
 #pragma unroll
-  for (int p = 0; p < kNormPasses; ++p) {
+  for (int p = 0; p < PASSES; ++p) {
     const uint32_t q[4] = {v[p].x, v[p].y, v[p].z, v[p].w};
 #pragma unroll
     for (int j = 0; j < 4; ++j) ss = fmaf(bf16hi(q[j]), bf16hi(q[j]), fmaf(bf16lo(q[j]), bf16lo(q[j]), ss));
   }
   const float r = rsqrtf(block_sum(ss, part) / static_cast<float>(H) + eps);
 #pragma unroll
-  for (int p = 0; p < kNormPasses; ++p) {
+  for (int p = 0; p < PASSES; ++p) {
     const int i = 8 * (kNormThreads * p + static_cast<int>(threadIdx.x));
     const uint32_t q[4] = {v[p].x, v[p].y, v[p].z, v[p].w};
     const uint32_t u[4] = {w[p].x, w[p].y, w[p].z, w[p].w};
@@ -237,9 +243,12 @@ hipError_t launch_rmsnorm(const uint16_t* x, int64_t rows, int64_t H, const uint
   if (rows <= 0) return hipSuccess;
   const uintptr_t bits = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out) |
                          reinterpret_cast<uintptr_t>(weight);  // (NULL weight: ones)
-  if (H % 8 == 0 && H <= 8 * kNormThreads * kNormPasses && (bits & 15u) == 0)
-    hipLaunchKernelGGL(rmsnorm_vec_kernel, dim3(static_cast<unsigned>(rows)), dim3(kNormThreads), 0, stream, x,
-                       static_cast<int>(H), weight, eps, out);
+  if (H % 8 == 0 && H >= 128 && H <= 8 * kNormThreads * kNormPasses && (bits & 15u) == 0)
+    hipLaunchKernelGGL(H <= 8 * kNormThreads       ? rmsnorm_vec_kernel<1>
+                       : H <= 2 * 8 * kNormThreads ? rmsnorm_vec_kernel<2>
+                                                   : rmsnorm_vec_kernel<kNormPasses>,
+                       dim3(static_cast<unsigned>(rows)), dim3(kNormThreads), 0, stream, x, static_cast<int>(H), weight,
+                       eps, out);
   else
     hipLaunchKernelGGL(rmsnorm_kernel, dim3(static_cast<unsigned>(rows)), dim3(kNormThreads), 0, stream, x, H, weight,
                        eps, out);
