@@ -65,7 +65,8 @@ enum {
   UQM_OPT_FUSED_DECODE = 1,   /* 1 (default): blocks of one or two tokens use the fused persistent
                                   kernel, one launch per token */
   UQM_OPT_MFMA_MIN_TOKENS = 3,     /* token count from which multi-token calls run the expert projections
-                                      as MFMA grouped GEMMs (default 2; 0 = never, batched GEMV instead) */
+                                      as MFMA grouped GEMMs (default 2; 0 = never, batched GEMV instead);
+                                      linears of at least as many rows may take MFMA tiles */
   UQM_OPT_OVERLAP_SHARED = 4,      /* 1 (default): multi-token blocks run the shared expert on a
                                       library-owned side stream (one per device, default priority),
                                       forked from and joined back into the caller's stream with
@@ -124,6 +125,8 @@ size_t uqm_moe_workspace_bytes(int64_t tokens, int64_t hidden_size, int64_t inte
                                int64_t shared_intermediate_size, int64_t num_experts, int64_t top_k);
 
 /* output[rows, out] = bf16(input[rows, in] @ dequant(W)^T), FP32 accumulation.
+ * Calls of few and of many rows (from 17 for Q8, 25 for Q4 and BF16) sum in
+ * different orders, so a row's result may differ in its last bit between them.
  * Replaces q4_linear: src/uma_qmoe/native/packed_q4_binding.cpp:130-163
  * (kernel packed_q4_kernel.cu:72-113, launcher :1430-1456). */
 int uqm_q4_linear(const void* input, int64_t rows, const void* packed, const float* scales,

@@ -16,6 +16,7 @@ from oracle import codec as oc
 from oracle import moe as om
 from test_gpu_kernels import assert_bf16_rounded
 from test_gpu_mfma import DEV, RAGGED, close, dense_cpu, layout_of, mfma_on, note, to_dev  # noqa: F401
+from uma_qmoe_amd import _native
 from uma_qmoe_amd import synthetic as syn
 
 pytestmark = pytest.mark.gpu
@@ -137,6 +138,32 @@ def test_linear_many_rows(hip_ext, encoding, rows, n, k):
         deq = data[0].float().numpy()
         got = hip_ext.bf16_linear(xd, wd)
     assert_bf16_rounded(got, x.float() @ torch.from_numpy(deq).T, "linear")
+
+
+@pytest.mark.parametrize("encoding", ["q4_group128", "q8_group128", "bf16_le"])
+def test_linear_obeys_the_mfma_option(hip_ext, encoding):
+    """With UQM_OPT_MFMA_MIN_TOKENS 0 (or above the rows) a linear of many rows
+    is the GEMV: bit for bit its rows in calls of four."""
+    note(f"linear option {encoding}")
+    rows, n, k = 136, 256, 2048
+    g = torch.Generator().manual_seed(8)
+    data, scales = syn.encode_projection(torch.randn(1, n, k, generator=g) * 0.02, encoding)
+    w, s = data[0].to(DEV), None if scales is None else scales[0].to(DEV)
+    x = torch.randn(rows, k, generator=g).to(torch.bfloat16).to(DEV)
+
+    def linear(v):
+        if encoding == "bf16_le":
+            return hip_ext.bf16_linear(v, w)
+        return (hip_ext.q4_linear if encoding == "q4_group128" else hip_ext.q8_linear)(v, w, s, n, k, 128)
+
+    gemv = torch.cat([linear(x[i:i + 4]) for i in range(0, rows, 4)])
+    assert not torch.equal(linear(x), gemv)  # the tiles sum in another order
+    try:
+        for least in (0, rows + 1):
+            hip_ext.set_option(_native.UQM_OPT_MFMA_MIN_TOKENS, least)
+            assert torch.equal(linear(x), gemv), least
+    finally:
+        hip_ext.set_option(_native.UQM_OPT_MFMA_MIN_TOKENS, 2)
 
 
 @pytest.mark.parametrize("which,t", [("ragged", 4300), ("ragged", 9700), ("c2", 2100)])

@@ -691,7 +691,10 @@ static int linear_impl(int enc, const void* input, int64_t rows, const void* w, 
   // up to ~300). Measured, us per call, 1408 x 2048: Q4 16 rows 12.2 vs 10.8, 24
   // 12.1 vs 14.6, 137 12.9 vs 71; Q8 16 13.5 vs 13.8, 137 vs 100; BF16 24 16.0 vs
   // 17.2, 137 vs 91; 768 x 2048: Q4 20 12.1 vs 10.9, 24 12.2 vs 12.6.
-  if (rows >= (enc == UQM_Q8 ? 17 : 25) && rows <= 0x7FFFFFFF && reinterpret_cast<uintptr_t>(output) % 8 == 0 &&
+  // UQM_OPT_MFMA_MIN_TOKENS rules them as the expert projections (0: always GEMV).
+  const int64_t min_rows = g_opt_mfma_min_tokens.load(std::memory_order_relaxed);
+  if (min_rows > 0 && rows >= min_rows && rows >= (enc == UQM_Q8 ? 17 : 25) && rows <= 0x7FFFFFFF &&
+      reinterpret_cast<uintptr_t>(output) % 8 == 0 &&
       prefill_supported(enc, out_features, in_features, group_size, rows, in_features)) {
     const int64_t row_blocks = (out_features + 127) / 128;
     const int64_t fewest = (rows + kPrefillTileTokens - 1) / kPrefillTileTokens;
