@@ -92,6 +92,36 @@ def test_infinities_and_nan_stay_in_their_token(mfma_on):  # noqa: F811
     assert out[0].isnan().all() and not out[7].isfinite().all()
 
 
+def test_silu_of_large_negative_gates(mfma_on):  # noqa: F811
+    """g / (1 + exp(-g)) down to the largest finite exp(-g) (g = -88.5), where
+    the reciprocal of 1 + exp(-g) is subnormal. Token t's gate is GATES[t % 8]
+    in every row, its up value 2^100; row 0 of the down matrix picks one of
+    them. The product keeps FP32's accuracy (exp's argument error included,
+    below 1e-4), then bf16 rounds it and the output: 2^-7 relative. Where
+    exp(-g) overflows the quotient is 0."""
+    note("prefill silu of large negative gates")
+    gates = torch.tensor([-80.0, -87.0, -87.5, -88.0, -88.5, -0.5, -89.0, -100.0])
+    shape = syn.MoEShape("prefill_silu", 256, 2, 1, 256, encoding="bf16_le")
+    t = 80
+    x = torch.zeros(t, 256, dtype=torch.bfloat16)
+    x[torch.arange(t), torch.arange(t) % 8] = 1
+    gate = torch.zeros(2, 256, 256)
+    gate[:, :, :8] = gates
+    up = torch.zeros(2, 256, 256)
+    up[:, :, :8] = 2.0 ** 100
+    down = torch.zeros(2, 256, 256)
+    down[:, 0, 17] = 1
+    layer = replace(syn.build_experts(shape), gate=gate.to(torch.bfloat16), up=up.to(torch.bfloat16),
+                    down=down.to(torch.bfloat16))
+    idx = (torch.arange(t) // 8 % 2).view(-1, 1)
+    got = mfma_on.moe_forward(to_dev(layer), x.to(DEV), idx.to(DEV), torch.ones(t, 1, dtype=torch.bfloat16, device=DEV))
+    g = gates.double()
+    ref = g / (1 + torch.exp(-g)) * 2.0 ** 100
+    out = got.cpu().double()[:, 0].view(-1, 8)
+    assert ((out[:, :6] - ref[:6]).abs() <= 2.0 ** -7 * ref[:6].abs()).all(), out[0]
+    assert (out[:, 6:].abs() <= ref[6:].abs()).all()
+
+
 def test_block_replays_from_a_graph(mfma_on):  # noqa: F811
     """A whole block on the large tiles, captured and replayed with eager work
     in between, equals the eager call bit for bit."""

@@ -161,14 +161,25 @@ __device__ __forceinline__ int row_swizzle(int r) {
   return ENC == kQ4 ? ((r & 11) | ((r >> 1) & 4)) : (r & 15);
 }
 
-// g / (1 + exp(-g)): the reciprocal refined by one Newton step, as accurate as
-// the divide at half its instructions. Where exp overflows (g below -88) the
-// reciprocal is 0 and the step's NaN becomes 1, so the result is -0 as with
-// the divide (NaN for -inf).
-__device__ __forceinline__ float silu_newton(float g) {
-  const float d = 1.0f + __expf(-g);
-  const float r = __builtin_amdgcn_rcpf(d);
-  return g * fmaf(fminf(fmaf(-d, r, 1.0f), 1.0f), r, r);
+// g / (1 + exp(-g)) of four values: the reciprocal refined by one Newton step,
+// as accurate as the divide at half its instructions. The reciprocal flushes
+// subnormal results: from 1 + exp(-g) = 2^126 on (g below -87.3) the wave
+// divides, for all four values (one comparison for the four and a branch that
+// is hardly ever taken).
+__device__ __forceinline__ f32x4_t silu4(f32x4_t g) {
+  f32x4_t d, s;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) d[e] = 1.0f + __expf(-g[e]);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float r = __builtin_amdgcn_rcpf(d[e]);
+    s[e] = g[e] * fmaf(fmaf(-d[e], r, 1.0f), r, r);
+  }
+  if (__builtin_expect(__any(fmaxf(fmaxf(d[0], d[1]), fmaxf(d[2], d[3])) > 0x1p126f), 0)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] = g[e] / d[e];
+  }
+  return s;
 }
 
 // s_waitcnt with only vmcnt limited (gfx9 encoding: vmcnt bits 3:0 and 15:14).
@@ -431,13 +442,15 @@ __device__ __forceinline__ void run_item(const MfmaArgs& a, unsigned char* lds, 
     if constexpr (MODE == kModeSilu) {
       const int r0 = rb * 64 + 16 * wave + 4 * q;
       if (r0 >= rows) continue;
-      uint32_t h[2];
+      uint32_t g2[2], u2[2], h[2];
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
-        const uint32_t g2 = pack_bf16x2(kUnit * acc[0][tt][2 * e], kUnit * acc[0][tt][2 * e + 1]);
-        const uint32_t u2 = pack_bf16x2(kUnit * acc[1][tt][2 * e], kUnit * acc[1][tt][2 * e + 1]);
-        h[e] = pack_bf16x2(silu_newton(bf16lo(g2)) * bf16lo(u2), silu_newton(bf16hi(g2)) * bf16hi(u2));
+        g2[e] = pack_bf16x2(kUnit * acc[0][tt][2 * e], kUnit * acc[0][tt][2 * e + 1]);
+        u2[e] = pack_bf16x2(kUnit * acc[1][tt][2 * e], kUnit * acc[1][tt][2 * e + 1]);
       }
+      const f32x4_t s = silu4(f32x4_t{bf16lo(g2[0]), bf16hi(g2[0]), bf16lo(g2[1]), bf16hi(g2[1])});
+#pragma unroll
+      for (int e = 0; e < 2; ++e) h[e] = pack_bf16x2(s[2 * e] * bf16lo(u2[e]), s[2 * e + 1] * bf16hi(u2[e]));
       *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + at + r0) = make_uint2(h[0], h[1]);
     } else {
 #pragma unroll
