@@ -278,6 +278,40 @@ def test_48_route_tiles(mfma_on):
     close(got, got_g, "48-route tiles mfma vs gemv", rel=5e-3, mx=1e-2)
 
 
+def random_experts(encoding, e, hidden, inter, seed):
+    """Experts of uniformly random codes with a standard deviation of about
+    0.02, made on the GPU (large shapes)."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+
+    def matrix(rows, cols):
+        top = 7 if encoding == "q4_group128" else 127
+        codes = torch.randint(-top, top + 1, (e, rows, cols), generator=g, device=DEV, dtype=torch.int8)
+        scales = 0.034 / top * (0.5 + torch.rand(e, rows * cols // 128, generator=g, device=DEV))
+        if encoding == "q4_group128":
+            codes = (codes[..., 0::2] & 15 | codes[..., 1::2] << 4).view(torch.uint8)
+        return codes, scales
+
+    (gate, gs), (up, us), (down, ds) = matrix(inter, hidden), matrix(inter, hidden), matrix(hidden, inter)
+    return DeviceExperts(encoding, 128, e, hidden, inter, gate, gs, up, us, down, ds)
+
+
+@pytest.mark.parametrize("encoding,e,k,t,hidden,inter", [("q4_group128", 44, 4, 198, 4096, 768),
+                                                         ("q8_group128", 4, 2, 36, 5248, 768)])
+def test_long_rows(mfma_on, encoding, e, k, t, hidden, inter):
+    """18 routes per expert and rows so long that their scales leave no LDS for
+    the widest items: Q4 4096 (no 128-row items), Q8 5248 (no 32-route tiles).
+    Sampled tokens against the oracle."""
+    note(f"mfma long rows {encoding}")
+    layer = random_experts(encoding, e, hidden, inter, 3)
+    shape = syn.MoEShape("long_rows", hidden, e, k, inter, encoding=encoding)
+    x = syn.hidden_states(shape, t, seed=8)
+    idx, w = routes(t, k, e, 21)
+    got = mfma_on.moe_forward(layer, x.to(DEV), idx.to(DEV), w.to(DEV)).cpu()
+    pick = torch.tensor([0, t // 2, t - 1])
+    ref = om.streaming_reference(x[pick], idx[pick], w[pick], 0, syn.DeviceLayerReader({0: layer}), num_experts=e)
+    close(got[pick], ref, f"long rows {encoding}", mx=2e-2 * max(1.0, ref.abs().max().item()))
+
+
 # K / 128 odd in both projections (H = 1152: 9 scale groups, I = 896: 7)
 ODD = syn.MoEShape("odd_k", 1152, 40, 4, 896)
 

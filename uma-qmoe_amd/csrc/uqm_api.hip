@@ -190,11 +190,14 @@ int nb_for(int enc, double mean_routes) {
 // Enough work items (row block x route tile) for the persistent grid: 8 MMA
 // waves (128 rows per item) when there is plenty of work, 4 (64 rows), then
 // waves and workgroups along K when there is little. Every K range keeps
-// >= 3 steps of 128 per wave.
-MfmaPlan plan_mfma(int enc, int nmat, int64_t rows, int64_t K, int nb, int64_t tiles, int cus, int max_split) {
+// >= 3 steps of 128 per wave. The scales of 128 long rows can leave no LDS for
+// the 8-wave ring (Q4 gate/up beyond K = 2432 with 32-route tiles): 4 waves then.
+MfmaPlan plan_mfma(int enc, int nmat, int64_t rows, int64_t K, int64_t group, int nb, int64_t tiles, int cus,
+                   int max_split) {
   MfmaPlan p;
   p.nb = nb;
-  if (nb <= 3 && (nmat == 1 || enc == UQM_Q4) && rows % 128 == 0 && rows / 128 * tiles >= cus) {
+  if (nb <= 3 && (nmat == 1 || enc == UQM_Q4) && rows % 128 == 0 && rows / 128 * tiles >= cus &&
+      uqm::mfma_fits(enc, nmat, rows, K, group, nb, 1, 8, 1)) {
     p.mw = 8;
     return p;
   }
@@ -208,6 +211,23 @@ MfmaPlan plan_mfma(int enc, int nmat, int64_t rows, int64_t K, int nb, int64_t t
   if (ks > max_split) ks = max_split;
   if (ks > max_by_k) ks = max_by_k;
   p.ksplit = ks < 1 ? 1 : static_cast<int>(ks);
+  return p;
+}
+
+// The grouped GEMMs of routed calls with `active` experts in tiles of 16 * nb
+// routes, and whether the kernel has both.
+struct RoutedPlan {
+  MfmaPlan gate_up, down;
+  bool fits;
+};
+RoutedPlan plan_routed(const uqm_expert_weights* w, int nb, int64_t active, int64_t T) {
+  const int64_t H = w->hidden_size, I = w->intermediate_size, g = w->group_size;
+  const int enc = w->encoding, cus = device_cus();
+  RoutedPlan p;
+  p.gate_up = plan_mfma(enc, 2, I, H, g, nb, active, cus, 1);
+  p.down = plan_mfma(enc, 1, H, I, g, nb, active, cus, T > 1 ? kMaxSplit : 1);
+  p.fits = uqm::mfma_fits(enc, 2, I, H, g, nb, p.gate_up.kw, p.gate_up.mw, 1) &&
+           uqm::mfma_fits(enc, 1, H, I, g, nb, p.down.kw, p.down.mw, p.down.ksplit);
   return p;
 }
 
@@ -272,13 +292,12 @@ int routed_tile_tokens(const uqm_expert_weights* w, bool shared, int64_t T, int6
   if (!routed_uses_mfma(w, T)) return 0;
   // 48-route tiles when most experts would otherwise take a second, nearly
   // empty 32-route tile (every tile costs a full pass over the expert's rows)
-  // and both Q4 projections run 128-row items (the only kernels built for them)
-  const int cus = device_cus();
-  if (mean > 32 && mean <= 48 && w->encoding == UQM_Q4 && w->intermediate_size % 128 == 0 &&
-      w->hidden_size % 128 == 0 && active * (w->intermediate_size / 128) >= cus &&
-      active * (w->hidden_size / 128) >= cus)
-    return 48;
-  return 16 * (mean >= 16 ? 2 : nb_for(w->encoding, mean));
+  // and both Q4 projections run 128-row items (the only kernels built for them);
+  // smaller tiles where the rows' scales leave no LDS for the larger ones
+  if (mean > 32 && mean <= 48 && w->encoding == UQM_Q4 && plan_routed(w, 3, active, T).fits) return 48;
+  for (int nb = mean >= 16 ? 2 : 1; nb >= 1; --nb)
+    if (plan_routed(w, nb, active, T).fits) return 16 * nb;
+  return 0;
 }
 
 // Per-device side stream and fork/join events: a multi-token block runs the
@@ -460,7 +479,8 @@ int run_routed(const uqm_expert_weights* w, const uint16_t* hidden, int64_t T, i
     g.order = kOrderAuto;
     g.active_count = at<int32_t>(ws, L.counters);
     const bool prefill = tile_tokens == kPrefillTileTokens;
-    const MfmaPlan pg = plan_mfma(w->encoding, 2, I, H, nb, active, cus, 1);
+    const RoutedPlan plan = prefill ? RoutedPlan{} : plan_routed(w, nb, active, T);
+    const MfmaPlan& pg = plan.gate_up;
     int rc = hip_check(prefill ? launch_prefill_mfma(w->encoding, 2, kModeSilu, g, stream)
                                : launch_expert_mfma(w->encoding, 2, g, pg.nb, pg.kw, pg.mw, cus, stream),
                        "gate/up MFMA launch");
@@ -480,7 +500,7 @@ int run_routed(const uqm_expert_weights* w, const uint16_t* hidden, int64_t T, i
     d.part_stride = R * H;
     d.order = kOrderRowFastest;
     if (prefill) return hip_check(launch_prefill_mfma(w->encoding, 1, kModeF32, d, stream), "down MFMA launch");
-    const MfmaPlan pd = plan_mfma(w->encoding, 1, H, I, nb, active, cus, T > 1 ? kMaxSplit : 1);
+    const MfmaPlan& pd = plan.down;
     d.ksplit = pd.ksplit;
     *parts = pd.ksplit;
     return hip_check(launch_expert_mfma(w->encoding, 1, d, pd.nb, pd.kw, pd.mw, cus, stream), "down MFMA launch");
@@ -593,7 +613,7 @@ int run_shared(const uqm_layer_weights* layer, const uint16_t* x, int64_t T, int
     g.out = at<uint16_t>(ws, L.h_shared);
     g.ldo = Is;
     g.ksplit = 1;
-    const MfmaPlan pg = plan_mfma(UQM_BF16, 2, Is, H, nb, tiles, cus, 1);
+    const MfmaPlan pg = plan_mfma(UQM_BF16, 2, Is, H, 0, nb, tiles, cus, 1);
     int rc = hip_check(launch_expert_mfma(UQM_BF16, 2, g, pg.nb, pg.kw, pg.mw, cus, stream), "shared gate/up MFMA launch");
     if (rc) return rc;
     MfmaArgs d = g;
@@ -606,7 +626,7 @@ int run_shared(const uqm_layer_weights* layer, const uint16_t* x, int64_t T, int
     d.out = at<float>(ws, L.y_shared);
     d.ldo = H;
     d.part_stride = T * H;
-    const MfmaPlan pd = plan_mfma(UQM_BF16, 1, H, Is, nb, tiles, cus, T > 1 ? kMaxSplit : 1);
+    const MfmaPlan pd = plan_mfma(UQM_BF16, 1, H, Is, 0, nb, tiles, cus, T > 1 ? kMaxSplit : 1);
     d.ksplit = pd.ksplit;
     *parts = pd.ksplit;
     return hip_check(launch_expert_mfma(UQM_BF16, 1, d, pd.nb, pd.kw, pd.mw, cus, stream), "shared down MFMA launch");

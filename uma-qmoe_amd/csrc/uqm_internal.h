@@ -101,6 +101,9 @@ bool mfma_supported(int enc, int64_t rows, int64_t K, int64_t group);
 // 16 * mw / kw rows); cus: compute units (the grid is persistent).
 hipError_t launch_expert_mfma(int enc, int nmat, const MfmaArgs& a, int nb, int kw, int mw, int cus,
                               hipStream_t stream);
+// Whether launch_expert_mfma takes that launch shape for rows (per expert) x K
+// matrices: long rows with many scales leave no LDS for the widest tiles.
+bool mfma_fits(int enc, int nmat, int64_t rows, int64_t K, int64_t group, int nb, int kw, int mw, int ksplit);
 
 // Route tables produced on the device by the top-k / permutation kernels.
 struct RouteTables {

@@ -674,11 +674,12 @@ int blocks_per_cu(size_t lds) {
 }
 
 template <int ENC, int NMAT, int MW, int NB, int KW>
-hipError_t launch_cfg(const MfmaArgs& args, int cus, hipStream_t stream) {
+hipError_t launch_cfg(const MfmaArgs& args, int cus, bool dry, hipStream_t stream) {
   using C = MfmaCfg<ENC, NMAT, MW, NB, KW>;
   MfmaArgs a = args;
   a.row_blocks = static_cast<int32_t>(a.rows / C::WGR);
   if (!cfg_fits<ENC, NMAT, MW, NB, KW>(a)) return hipErrorInvalidValue;
+  if (dry) return hipSuccess;
   const size_t lds = lds_bytes_for<ENC, NMAT, MW, NB, KW>(a.K, a.group);
   constexpr int MODE = NMAT == 2 ? kModeSilu : kModeF32;
   auto kernel = expert_mfma_kernel<ENC, NMAT, MW, NB, KW, MODE>;
@@ -700,20 +701,20 @@ hipError_t launch_cfg(const MfmaArgs& args, int cus, hipStream_t stream) {
 }
 
 template <int ENC, int NMAT, int MW, int KW>
-hipError_t launch_nb(const MfmaArgs& a, int nb, int cus, hipStream_t stream) {
-  if (nb <= 1) return launch_cfg<ENC, NMAT, MW, 1, KW>(a, cus, stream);
+hipError_t launch_nb(const MfmaArgs& a, int nb, int cus, bool dry, hipStream_t stream) {
+  if (nb <= 1) return launch_cfg<ENC, NMAT, MW, 1, KW>(a, cus, dry, stream);
   if constexpr (KW == 1) {
-    if (nb <= 2) return launch_cfg<ENC, NMAT, MW, 2, KW>(a, cus, stream);
+    if (nb <= 2) return launch_cfg<ENC, NMAT, MW, 2, KW>(a, cus, dry, stream);
     if constexpr (MW == 8) {
       // 48-route tiles; the kernel's tile size must equal the tile list's
-      if (nb == 3) return launch_cfg<ENC, NMAT, MW, 3, KW>(a, cus, stream);
+      if (nb == 3) return launch_cfg<ENC, NMAT, MW, 3, KW>(a, cus, dry, stream);
     }
     if constexpr (MW == 4) {
       if (nb == 3) return hipErrorInvalidValue;
-      if (nb <= 4) return launch_cfg<ENC, NMAT, MW, 4, KW>(a, cus, stream);
+      if (nb <= 4) return launch_cfg<ENC, NMAT, MW, 4, KW>(a, cus, dry, stream);
       // 128-route tiles exist for BF16 only (a smaller kernel tile would drop routes)
       if constexpr (ENC == kBF16) {
-        if (nb <= 8) return launch_cfg<ENC, NMAT, MW, 8, KW>(a, cus, stream);
+        if (nb <= 8) return launch_cfg<ENC, NMAT, MW, 8, KW>(a, cus, dry, stream);
       }
     }
   }
@@ -721,17 +722,17 @@ hipError_t launch_nb(const MfmaArgs& a, int nb, int cus, hipStream_t stream) {
 }
 
 template <int ENC>
-hipError_t launch_enc(int nmat, const MfmaArgs& a, int nb, int kw, int mw, int cus, hipStream_t stream) {
+hipError_t launch_enc(int nmat, const MfmaArgs& a, int nb, int kw, int mw, int cus, bool dry, hipStream_t stream) {
   if (nmat == 2) {
-    if (kw == 4) return launch_nb<ENC, 2, 4, 4>(a, nb, cus, stream);
+    if (kw == 4) return launch_nb<ENC, 2, 4, 4>(a, nb, cus, dry, stream);
     if constexpr (ENC == kQ4) {  // Q8/BF16 gate+up tiles need too many registers for 8 MMA waves
-      if (mw == 8) return launch_nb<ENC, 2, 8, 1>(a, nb, cus, stream);
+      if (mw == 8) return launch_nb<ENC, 2, 8, 1>(a, nb, cus, dry, stream);
     }
-    return launch_nb<ENC, 2, 4, 1>(a, nb, cus, stream);
+    return launch_nb<ENC, 2, 4, 1>(a, nb, cus, dry, stream);
   }
-  if (kw == 4) return launch_nb<ENC, 1, 4, 4>(a, nb, cus, stream);
-  if (mw == 8) return launch_nb<ENC, 1, 8, 1>(a, nb, cus, stream);
-  return launch_nb<ENC, 1, 4, 1>(a, nb, cus, stream);
+  if (kw == 4) return launch_nb<ENC, 1, 4, 4>(a, nb, cus, dry, stream);
+  if (mw == 8) return launch_nb<ENC, 1, 8, 1>(a, nb, cus, dry, stream);
+  return launch_nb<ENC, 1, 4, 1>(a, nb, cus, dry, stream);
 }
 
 // Q4 gate/up tiles of 16 routes on the wide form (K-steps of two scale
@@ -742,14 +743,15 @@ hipError_t launch_enc(int nmat, const MfmaArgs& a, int nb, int kw, int mw, int c
 // c5 109.4 vs 97.9 with one workgroup per CU instead of two, batch 32 +1 us
 // with K = 1408, whose odd group count left one step half used) and wider
 // gate/up tiles (their rings do not fit).
-hipError_t launch_q4_wide(int nmat, const MfmaArgs& a, int nb, int kw, int mw, int cus, hipStream_t stream) {
+hipError_t launch_q4_wide(int nmat, const MfmaArgs& a, int nb, int kw, int mw, int cus, bool dry,
+                          hipStream_t stream) {
   if (nmat != 2 || nb != 1 || kw != 1 || a.group % 128 != 0 || a.K % 256 != 0) return hipErrorNotSupported;
   if (mw == 8) {
     if (!cfg_fits<kQ4Wide, 2, 8, 1, 1>(a)) return hipErrorNotSupported;
-    return launch_cfg<kQ4Wide, 2, 8, 1, 1>(a, cus, stream);
+    return launch_cfg<kQ4Wide, 2, 8, 1, 1>(a, cus, dry, stream);
   }
   if (!cfg_fits<kQ4Wide, 2, 4, 1, 1>(a)) return hipErrorNotSupported;
-  return launch_cfg<kQ4Wide, 2, 4, 1, 1>(a, cus, stream);
+  return launch_cfg<kQ4Wide, 2, 4, 1, 1>(a, cus, dry, stream);
 }
 
 }  // namespace
@@ -760,8 +762,11 @@ bool mfma_supported(int enc, int64_t rows, int64_t K, int64_t group) {
   return group > 0 && group % 128 == 0 && K % group == 0 && K / group <= 64;
 }
 
-hipError_t launch_expert_mfma(int enc, int nmat, const MfmaArgs& args, int nb, int kw, int mw, int cus,
-                              hipStream_t stream) {
+namespace {
+
+// Checks the launch shape and launches, or (dry) only checks it.
+hipError_t expert_mfma(int enc, int nmat, const MfmaArgs& args, int nb, int kw, int mw, int cus, bool dry,
+                       hipStream_t stream) {
   MfmaArgs a = args;
   if (a.ksplit < 1) a.ksplit = 1;
   if (nmat == 2 && a.ksplit != 1) return hipErrorInvalidValue;
@@ -773,15 +778,31 @@ hipError_t launch_expert_mfma(int enc, int nmat, const MfmaArgs& args, int nb, i
   if (a.rows % wgr != 0) return hipErrorInvalidValue;
   if ((a.w_tail != nullptr || (a.rows_valid > 0 && a.rows_valid != a.rows)) && wgr != 16) return hipErrorInvalidValue;
   if (enc != kBF16) a.scales_per_expert = (a.rows * a.K + a.group - 1) / a.group;
-  if (a.tile_bound <= 0) return hipSuccess;
+  if (!dry && a.tile_bound <= 0) return hipSuccess;
   if (cus < 8) cus = 8;
   if (enc == kQ4) {
-    const hipError_t e = launch_q4_wide(nmat, a, nb, kw, mw, cus, stream);
+    const hipError_t e = launch_q4_wide(nmat, a, nb, kw, mw, cus, dry, stream);
     if (e != hipErrorNotSupported) return e;
   }
-  if (enc == kQ4) return launch_enc<kQ4>(nmat, a, nb, kw, mw, cus, stream);
-  if (enc == kQ8) return launch_enc<kQ8>(nmat, a, nb, kw, mw, cus, stream);
-  return launch_enc<kBF16>(nmat, a, nb, kw, mw, cus, stream);
+  if (enc == kQ4) return launch_enc<kQ4>(nmat, a, nb, kw, mw, cus, dry, stream);
+  if (enc == kQ8) return launch_enc<kQ8>(nmat, a, nb, kw, mw, cus, dry, stream);
+  return launch_enc<kBF16>(nmat, a, nb, kw, mw, cus, dry, stream);
+}
+
+}  // namespace
+
+hipError_t launch_expert_mfma(int enc, int nmat, const MfmaArgs& a, int nb, int kw, int mw, int cus,
+                              hipStream_t stream) {
+  return expert_mfma(enc, nmat, a, nb, kw, mw, cus, false, stream);
+}
+
+bool mfma_fits(int enc, int nmat, int64_t rows, int64_t K, int64_t group, int nb, int kw, int mw, int ksplit) {
+  MfmaArgs a{};
+  a.rows = rows;
+  a.K = K;
+  a.group = group;
+  a.ksplit = ksplit;
+  return expert_mfma(enc, nmat, a, nb, kw, mw, 256, true, nullptr) == hipSuccess;
 }
 
 }  // namespace uqm
