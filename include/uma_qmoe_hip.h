@@ -204,6 +204,25 @@ int uqm_norm_moe_layer(const uqm_layer_weights* layer, const void* hidden, int64
                        float eps, void* output, void* logits, void* routing_weights, int64_t* expert_indices,
                        void* workspace, size_t workspace_bytes, void* stream);
 
+/* Kernels a call takes (uqm_moe_layer_plan). */
+typedef struct uqm_layer_plan {
+  int32_t routed_tile;         /* routed projections: most routes per tile of the MFMA kernels (144: the
+                                  large-tile kernel; 48, 32, 16); 1: streaming GEMV; 0: staged GEMV;
+                                  -1: the fused kernel, one launch per token                        */
+  int32_t gate_up_rows;        /* shared expert on the dense kernel: weight rows (both matrices) and */
+  int32_t gate_up_tokens;      /* tokens per work item of its gate/up; 0 without it                  */
+  int32_t down_rows;           /* the same of its down projection                                    */
+  int32_t down_tokens;
+  int32_t down_split;          /* workgroups along K of its down projection                          */
+} uqm_layer_plan;
+
+/* Reports which kernels uqm_moe_layer with `layer` and `tokens` tokens runs
+ * under the current options (has_shared = 0: also uqm_moe_forward; the router
+ * and the device memory behind the pointers are not looked at). Host only:
+ * without a device it plans for 256 compute units. For tests and measurements
+ * that mean a particular kernel; no counterpart in the reference. */
+int uqm_moe_layer_plan(const uqm_layer_weights* layer, int64_t tokens, uqm_layer_plan* plan);
+
 /* Sets a process-wide option (UQM_OPT_*). No counterpart in the reference:
  * it selects between this library's own single-token code paths. */
 int uqm_set_option(int option, int64_t value);

@@ -257,39 +257,64 @@ bool routed_uses_stream(const uqm_expert_weights* w) {
 }
 
 // Whether the routed projections of T tokens take the large-tile kernel
-// (uqm_prefill.hip), from the mean routes per active expert: 25 for Q4 (40 with
-// a shared expert beside them), 22 for Q8, 4 for BF16. Its items convert a row
-// once for up to 144 routes and pad to 16; below, the conversion of a 32-row
-// wave outweighs its few MFMAs and the smaller tiles of uqm_mfma.hip are better
-// (BF16 converts nothing). Measured, large tiles against small (us per call;
-// Qwen shapes: whole block with its shared expert, OLMoE: whole block, Zipf: 128
-// experts, routed only):
+// (uqm_prefill.hip) rather than tiles of small_tile routes of uqm_mfma.hip (0:
+// the GEMV). Two conditions.
+//
+// Enough routes per active expert on average: 25 for Q4 (40 with a shared
+// expert beside them), 22 for Q8, 4 for BF16. Its items convert a row once for up
+// to 144 routes and pad to 16; below, the conversion of a 32-row wave outweighs
+// its few MFMAs and the smaller tiles of uqm_mfma.hip are better (BF16 converts
+// nothing). Measured, large tiles against small (us per call; Qwen shapes: whole
+// block with its shared expert, OLMoE: whole block, Zipf: 128 experts, routed
+// only):
 //   Q4   Qwen 34 routes 168 vs 160, 43 190 vs 216, 68 215 vs 306;
 //        OLMoE 20 96 vs 89, 25 99 vs 108; Zipf 20 119 vs 117, 25 123 vs 130
 //   Q8   Qwen 17 178 vs 175, 26 193 vs 195, 32 202 vs 233; Zipf 25 146 vs 182
 //   BF16 Qwen 5 231 vs 236, 20 256 vs 253, 32 276 vs 302; Zipf 4 114 vs 118,
 //        12 158 vs 194; OLMoE 4 169 vs 181
-bool routed_uses_prefill(const uqm_expert_weights* w, bool shared, int64_t T, int64_t R, double mean) {
+//
+// And enough items for the card, or enough work in them: the kernel has no K
+// split, which uqm_mfma.hip takes for few items, and an item is a serial chain of
+// K / 128 stages. Few experts make few items: the down projection's row blocks x
+// tiles must reach the CUs, or its row blocks x routes 12 (Q4), 18 (Q8) or 16
+// (BF16) per CU: the least mean loss against the better of both over 600 calls
+// of 4 to 24 experts from 1024 x 768 to 4096 x 4096 and 5 to 200 routes per
+// expert, 0.6% (all on large tiles 4.4%, none 15.6%). Gain over the small tiles
+// at that many items and routes per expert:
+//   256 and more  BF16 5 0.98-1.10, Q8 22 0.96-1.09, Q4 25 1.06-1.19
+//   128           BF16 24 0.84-0.91, 32 0.97-1.22; Q8 26 0.75-0.98, 40 1.0-1.20;
+//                 Q4 25 0.82-1.09, 32 1.02-1.29
+//   64            BF16 48 0.83-0.89, 64 0.92-1.10; Q8 64 0.84-1.07, 96 1.03-1.14;
+//                 Q4 48 0.93-1.03, 64 0.94-1.17
+//   32            64 0.84-0.99 all encodings, 200 (two tiles each) 1.15-1.32
+// Shapes that uqm_mfma.hip does not take gain at any size (256 x 256, 4 experts,
+// 16 routes 1.6, Q4 32 routes 5.4: the GEMV).
+bool routed_uses_prefill(const uqm_expert_weights* w, bool shared, int64_t T, int64_t R, int64_t active,
+                         int small_tile) {
   const int64_t min_t = g_opt_mfma_min_tokens.load(std::memory_order_relaxed);
   if (min_t <= 0 || T < min_t) return false;
+  const double mean = static_cast<double>(R) / static_cast<double>(active);
   const double least = w->encoding == UQM_Q4 ? (shared ? 40.0 : 25.0) : w->encoding == UQM_Q8 ? 22.0 : 4.0;
   if (mean < least) return false;
   const int64_t H = w->hidden_size, I = w->intermediate_size;
-  return uqm::prefill_supported(w->encoding, I, H, w->group_size, T, H) &&
-         uqm::prefill_supported(w->encoding, H, I, w->group_size, R, I);
+  if (!uqm::prefill_supported(w->encoding, I, H, w->group_size, T, H) ||
+      !uqm::prefill_supported(w->encoding, H, I, w->group_size, R, I))
+    return false;
+  if (small_tile == 0) return true;
+  const int64_t cus = device_cus(), row_blocks = (H + 127) / 128;
+  const int64_t most = active * uqm::kPrefillTileTokens;
+  const int64_t items = row_blocks * active * ((R + most - 1) / most);
+  const int64_t per_cu = w->encoding == UQM_Q4 ? 12 : w->encoding == UQM_Q8 ? 18 : 16;
+  return items >= cus || row_blocks * R >= per_cu * cus;
 }
 
-// Route tile size the routed MFMA path uses (0 = GEMV path). From 16 routes
-// per expert on average, 32-route tiles: measured faster than 16 (c5: 80 vs
-// 105 us) and than 64 (c4: 247 vs 271 us), whose 4-wave items take longer per
-// weight byte.
-int routed_tile_tokens(const uqm_expert_weights* w, bool shared, int64_t T, int64_t k) {
-  const int64_t R = T * k;
-  const int64_t active = R < w->num_experts ? R : w->num_experts;
-  const double mean = static_cast<double>(R) / static_cast<double>(active);
-  if (routed_uses_stream(w) && R <= g_opt_stream_max_routes.load(std::memory_order_relaxed)) return 0;
-  if (routed_uses_prefill(w, shared, T, R, mean)) return uqm::kPrefillTileTokens;
+// Route tile size of the routed projections on uqm_mfma.hip (0 = GEMV path).
+// From 16 routes per expert on average, 32-route tiles: measured faster than 16
+// (c5: 80 vs 105 us) and than 64 (c4: 247 vs 271 us), whose 4-wave items take
+// longer per weight byte.
+int grouped_tile_tokens(const uqm_expert_weights* w, int64_t T, int64_t R, int64_t active) {
   if (!routed_uses_mfma(w, T)) return 0;
+  const double mean = static_cast<double>(R) / static_cast<double>(active);
   // 48-route tiles when most experts would otherwise take a second, nearly
   // empty 32-route tile (every tile costs a full pass over the expert's rows)
   // and both Q4 projections run 128-row items (the only kernels built for them);
@@ -298,6 +323,23 @@ int routed_tile_tokens(const uqm_expert_weights* w, bool shared, int64_t T, int6
   for (int nb = mean >= 16 ? 2 : 1; nb >= 1; --nb)
     if (plan_routed(w, nb, active, T).fits) return 16 * nb;
   return 0;
+}
+
+// Route tile size the routed MFMA path uses (0 = GEMV path).
+int routed_tile_tokens(const uqm_expert_weights* w, bool shared, int64_t T, int64_t k) {
+  const int64_t R = T * k;
+  const int64_t active = R < w->num_experts ? R : w->num_experts;
+  if (routed_uses_stream(w) && R <= g_opt_stream_max_routes.load(std::memory_order_relaxed)) return 0;
+  const int small = grouped_tile_tokens(w, T, R, active);
+  return routed_uses_prefill(w, shared, T, R, active, small) ? uqm::kPrefillTileTokens : small;
+}
+
+// Whether a call of T tokens runs on the fused kernel, one launch per token.
+bool uses_fused(const uqm_expert_weights* w, int64_t Is, int64_t T, int64_t k) {
+  return T <= kFusedMaxTokens && g_opt_fused.load(std::memory_order_relaxed) != 0 &&
+         uqm::fused_config_id(w->encoding, w->hidden_size, w->intermediate_size, Is, k, w->num_experts) >= 0 &&
+         (w->encoding == UQM_BF16 ||
+          (w->hidden_size % w->group_size == 0 && w->intermediate_size % w->group_size == 0));
 }
 
 // Per-device side stream and fork/join events: a multi-token block runs the
@@ -551,6 +593,10 @@ int run_routed(const uqm_expert_weights* w, const uint16_t* hidden, int64_t T, i
                    "down launch");
 }
 
+// Compute units of the shared expert's persistent grids; beside the routing
+// chain 3/4 of them.
+int shared_cus(bool beside) { return beside ? device_cus() * 3 / 4 : device_cus(); }
+
 // Shared expert on T tokens: h_shared = silu(x Wg^T) * (x Wu^T), y_shared =
 // h_shared Wd^T (FP32, *parts K-split partials).
 int run_shared(const uqm_layer_weights* layer, const uint16_t* x, int64_t T, int64_t H, const Layout& L, void* ws,
@@ -561,7 +607,7 @@ int run_shared(const uqm_layer_weights* layer, const uint16_t* x, int64_t T, int
   if (shared_uses_dense(H, Is, T)) {
     // Dense square tiles (uqm_dense.hip); beside the routing chain at 3/4 of
     // the CUs, as the grouped kernel below.
-    const int cus = beside ? device_cus() * 3 / 4 : device_cus();
+    const int cus = shared_cus(beside);
     DenseArgs g{};
     g.w[0] = static_cast<const uint16_t*>(layer->shared_gate);
     g.w[1] = static_cast<const uint16_t*>(layer->shared_up);
@@ -599,7 +645,7 @@ int run_shared(const uqm_layer_weights* layer, const uint16_t* x, int64_t T, int
     // Beside the routing chain, the persistent grids take 3/4 of the CUs'
     // slots, so that the router and top-k launches find room at once (batch
     // 32: 113.6 vs 122.0 us per call; 1/2: 118.0, 5/8: 117.9, 7/8: 120.9).
-    const int cus = beside ? device_cus() * 3 / 4 : device_cus();
+    const int cus = shared_cus(beside);
     MfmaArgs g{};
     g.w[0] = static_cast<const uint8_t*>(layer->shared_gate);
     g.w[1] = static_cast<const uint8_t*>(layer->shared_up);
@@ -844,9 +890,7 @@ int uqm_moe_forward(const uqm_expert_weights* weights, const void* hidden, int64
   const int64_t H = weights->hidden_size, I = weights->intermediate_size, E = weights->num_experts;
   // One or two tokens: the fused single-token kernel with the caller's routes
   // (no router), one launch per token.
-  const bool fused = tokens <= kFusedMaxTokens && g_opt_fused.load(std::memory_order_relaxed) != 0 &&
-                     fused_config_id(weights->encoding, H, I, 0, top_k, E) >= 0 &&
-                     (weights->encoding == UQM_BF16 || (H % weights->group_size == 0 && I % weights->group_size == 0));
+  const bool fused = uses_fused(weights, 0, tokens, top_k);
   if ((rc = note_layout(workspace, L, {E, top_k, I, 0}, fused, s))) return rc;
   if (fused) {
     FusedArgs fa{};
@@ -947,9 +991,7 @@ int moe_layer_impl(const uqm_layer_weights* layer, const void* hidden, int64_t t
   // One or two tokens: one persistent launch per token for the whole block
   // (two tokens: 2 x 20.7 us against 57.9 us on the multi-launch path for c2
   // shapes; three: 62.1 against 63.1).
-  const bool fused = tokens <= kFusedMaxTokens && g_opt_fused.load(std::memory_order_relaxed) != 0 &&
-                     fused_config_id(w->encoding, H, w->intermediate_size, Is, k, E) >= 0 &&
-                     (w->encoding == UQM_BF16 || (H % w->group_size == 0 && w->intermediate_size % w->group_size == 0));
+  const bool fused = uses_fused(w, Is, tokens, k);
   if ((rc = note_layout(workspace, L, {E, k, w->intermediate_size, Is}, fused, s))) return rc;
   if (fused) {
     FusedArgs fa{};
@@ -1151,6 +1193,33 @@ int uqm_norm_moe_layer(const uqm_layer_weights* layer, const void* hidden, int64
                        void* workspace, size_t workspace_bytes, void* stream) {
   return moe_layer_impl(layer, hidden, tokens, InputNorm{true, norm_weight, eps}, output, logits, routing_weights,
                         expert_indices, workspace, workspace_bytes, stream);
+}
+
+int uqm_moe_layer_plan(const uqm_layer_weights* layer, int64_t tokens, uqm_layer_plan* plan) {
+  if (layer == nullptr || plan == nullptr) return fail(UQM_ERR_ARGUMENT, "layer or plan is NULL");
+  const uqm_expert_weights* w = &layer->experts;
+  int rc;
+  if ((rc = check_experts(w))) return rc;
+  const int64_t k = layer->top_k, Is = layer->has_shared ? layer->shared_intermediate_size : 0;
+  if (tokens <= 0 || k <= 0 || k > 64 || Is < 0) return fail(UQM_ERR_ARGUMENT, "need tokens > 0 and 1 <= top_k <= 64");
+  *plan = uqm_layer_plan{};
+  if (uses_fused(w, Is, tokens, k)) {
+    plan->routed_tile = -1;
+    return UQM_OK;
+  }
+  const int tile = routed_tile_tokens(w, layer->has_shared != 0, tokens, k);
+  plan->routed_tile = tile == 0 && routed_uses_stream(w) ? 1 : tile;
+  if (layer->has_shared && shared_uses_dense(w->hidden_size, Is, tokens)) {
+    const bool beside = g_opt_overlap_shared.load(std::memory_order_relaxed) != 0;
+    const uqm::DensePlan g = uqm::plan_dense(2, Is, w->hidden_size, tokens, shared_cus(beside), 1);
+    const uqm::DensePlan d = uqm::plan_dense(1, w->hidden_size, Is, tokens, shared_cus(beside), kMaxSplit);
+    plan->gate_up_rows = g.rows;
+    plan->gate_up_tokens = 32 * g.waves;
+    plan->down_rows = d.rows;
+    plan->down_tokens = 32 * d.waves;
+    plan->down_split = d.ksplit;
+  }
+  return UQM_OK;
 }
 
 int uqm_set_option(int option, int64_t value) {

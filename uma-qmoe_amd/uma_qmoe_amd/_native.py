@@ -76,6 +76,13 @@ class LayerWeights(ctypes.Structure):
     ]
 
 
+class LayerPlan(ctypes.Structure):
+    """uqm_layer_plan."""
+
+    _fields_ = [(name, _i32) for name in ("routed_tile", "gate_up_rows", "gate_up_tokens", "down_rows", "down_tokens",
+                                          "down_split")]
+
+
 class PackTensor(ctypes.Structure):
     """uqm_pack_tensor."""
 
@@ -127,6 +134,7 @@ SIGNATURES = {
         ctypes.c_int,
         (ctypes.POINTER(LayerWeights), _vp, _i64, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, ctypes.c_size_t, _vp),
     ),
+    "uqm_moe_layer_plan": (ctypes.c_int, (ctypes.POINTER(LayerWeights), _i64, ctypes.POINTER(LayerPlan))),
     "uqm_rmsnorm": (ctypes.c_int, (_vp, _i64, _i64, _vp, ctypes.c_float, _vp, _vp)),
     "uqm_dequantize": (ctypes.c_int, (_i32, _vp, _vp, _i64, _i64, _vp, _vp)),
     "uqm_set_option": (ctypes.c_int, (ctypes.c_int, _i64)),
