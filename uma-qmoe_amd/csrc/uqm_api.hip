@@ -618,7 +618,8 @@ int run_shared(const uqm_layer_weights* layer, const uint16_t* x, int64_t T, int
     g.T = T;
     g.out = at<uint16_t>(ws, L.h_shared);
     g.ldo = Is;
-    int rc = hip_check(launch_dense_mfma(2, g, plan_dense(2, Is, H, T, cus, 1), cus, stream), "shared gate/up dense launch");
+    int rc = hip_check(launch_dense_mfma(2, g, plan_dense(2, Is, H, T, cus, beside, 1), cus, stream),
+                       "shared gate/up dense launch");
     if (rc) return rc;
     DenseArgs d{};
     d.w[0] = static_cast<const uint16_t*>(layer->shared_down);
@@ -630,7 +631,7 @@ int run_shared(const uqm_layer_weights* layer, const uint16_t* x, int64_t T, int
     d.out = at<float>(ws, L.y_shared);
     d.ldo = H;
     d.part_stride = T * H;
-    const DensePlan pd = plan_dense(1, H, Is, T, cus, kMaxSplit);
+    const DensePlan pd = plan_dense(1, H, Is, T, cus, beside, kMaxSplit);
     *parts = pd.ksplit;
     return hip_check(launch_dense_mfma(1, d, pd, cus, stream), "shared down dense launch");
   }
@@ -1211,8 +1212,8 @@ int uqm_moe_layer_plan(const uqm_layer_weights* layer, int64_t tokens, uqm_layer
   plan->routed_tile = tile == 0 && routed_uses_stream(w) ? 1 : tile;
   if (layer->has_shared && shared_uses_dense(w->hidden_size, Is, tokens)) {
     const bool beside = g_opt_overlap_shared.load(std::memory_order_relaxed) != 0;
-    const uqm::DensePlan g = uqm::plan_dense(2, Is, w->hidden_size, tokens, shared_cus(beside), 1);
-    const uqm::DensePlan d = uqm::plan_dense(1, w->hidden_size, Is, tokens, shared_cus(beside), kMaxSplit);
+    const uqm::DensePlan g = uqm::plan_dense(2, Is, w->hidden_size, tokens, shared_cus(beside), beside, 1);
+    const uqm::DensePlan d = uqm::plan_dense(1, w->hidden_size, Is, tokens, shared_cus(beside), beside, kMaxSplit);
     plan->gate_up_rows = g.rows;
     plan->gate_up_tokens = 32 * g.waves;
     plan->down_rows = d.rows;

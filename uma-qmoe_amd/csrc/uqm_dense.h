@@ -33,13 +33,14 @@ bool dense_supported(int64_t rows, int64_t K, int64_t T);
 
 // Work item (4 or 8 waves: 128 or 256 tokens; 128 or, with 8 waves, 256 weight
 // rows, both matrices of gate/up together) and K split (kModeF32 only, at most
-// max_split) with the least estimated time on cus CUs.
+// max_split) with the least estimated time on cus CUs (beside: while the routing
+// chain uses what they leave idle).
 struct DensePlan {
   int waves;
   int rows;
   int ksplit;
 };
-DensePlan plan_dense(int nmat, int64_t rows, int64_t K, int64_t T, int cus, int max_split);
+DensePlan plan_dense(int nmat, int64_t rows, int64_t K, int64_t T, int cus, bool beside, int max_split);
 
 // nmat 2 = gate/up with the SiLU epilogue, 1 = FP32 rows; cus = compute units
 // the persistent grid may take.

@@ -340,19 +340,28 @@ hipError_t launch_cfg(const DenseArgs& a, int cus, hipStream_t stream) {
 
 }  // namespace
 
-DensePlan plan_dense(int nmat, int64_t rows, int64_t K, int64_t T, int cus, int max_split) {
-  // Relative time of one stage per item size: the 8-wave item (128 x 256) takes
-  // ~1.4 times as long per stage as the 4-wave one (128 x 128) for twice the
-  // work (c4 gate/up: 1.1 vs 0.79 us per stage), the 256 x 256 one ~2 times for
-  // four times (gate/up at 2048 tokens on 192 CUs 129 vs 145 us with 128 x 256).
-  // With 2.0 the block takes (us per call, against no 256-row items) 365 vs 398
-  // at 2048 tokens, 278 vs 286 at 1400, 192 vs 194 at 700; from 2.3 on the
-  // planner leaves 1400 and 1535 tokens on 128 rows (287 vs 278, 397 vs 383).
+DensePlan plan_dense(int nmat, int64_t rows, int64_t K, int64_t T, int cus, bool beside, int max_split) {
+  // Time per work item: K stages plus a fixed part (first loads, outputs), in
+  // stages of the 4-wave item (0.57 us). On their own on 192 CUs the three sizes
+  // take 1, 1.38 and 2.18 per stage and 8, 10 and 19 per item (gate/up with K =
+  // 2048 23.4, 31.7 and 51.7 us a round); beside the routing chain, whose loads and
+  // launches they overlap, a block's time follows 1, 1.34 and 2.1 and half of
+  // the fixed parts.
+  //   * A launch takes ceil(items / CUs) rounds of them. Beside the routing chain
+  //     the CUs that a last round leaves idle do other work, so that the round
+  //     counts for less (65% whole, 35% by its items), but for one item at least.
+  //   * Every part of a K split beyond the first is written and read once more
+  //     (2048 tokens of 2048: 5 to 7 us).
+  // Fitted to the times of 74 blocks under each of their 27 plans (32 and 60
+  // experts, shared expert 1408 to 6400 wide, hidden size 1024 to 4096, 128 to 4096
+  // tokens): 1.1% above the best plan on average; with 1.0, 1.4 and 2.0 per stage
+  // and nothing else 1.7%, and up to 10% (hidden 2048, shared 2816, 1025 tokens 155
+  // us per call against 141).
   struct Size {
     int waves, rows;
-    double stage;
+    double stage, item;
   };
-  const Size sizes[] = {{4, 128, 1.0}, {8, 128, 1.4}, {8, 256, 2.0}};
+  const Size sizes[] = {{4, 128, 1.0, 4.0}, {8, 128, 1.34, 5.0}, {8, 256, 2.1, 10.0}};
   const int64_t steps = K / kStepK;
   const int64_t grid = cus < 8 ? 8 : cus;
   DensePlan best{4, 128, 1};
@@ -360,8 +369,12 @@ DensePlan plan_dense(int nmat, int64_t rows, int64_t K, int64_t T, int cus, int 
   for (const Size& z : sizes) {
     for (int ks = 1; ks <= (nmat == 2 ? 1 : max_split); ks *= 2) {
       if (steps % ks != 0) continue;
-      const int64_t rounds = (dense_items(nmat, rows, T, z.waves, z.rows, ks) + grid - 1) / grid;
-      const double cost = static_cast<double>(rounds * (steps / ks)) * z.stage;
+      const int64_t items = dense_items(nmat, rows, T, z.waves, z.rows, ks);
+      const double whole = static_cast<double>((items + grid - 1) / grid);
+      const double even = static_cast<double>(items) / static_cast<double>(grid);
+      const double rounds = beside && whole > 1.0 ? 0.65 * whole + 0.35 * even : whole;
+      const double cost = rounds * (static_cast<double>(steps / ks) * z.stage + z.item) +
+                          3e-6 * static_cast<double>((ks - 1) * T * rows);
       if (best_cost < 0.0 || cost < best_cost) {  // ties: smaller items, smaller split
         best_cost = cost;
         best = DensePlan{z.waves, z.rows, ks};
