@@ -163,9 +163,12 @@ __device__ __forceinline__ int row_swizzle(int r) {
 
 // g / (1 + exp(-g)) of four values: the reciprocal refined by one Newton step,
 // as accurate as the divide at half its instructions. The reciprocal flushes
-// subnormal results: from 1 + exp(-g) = 2^126 on (g below -87.3) the wave
-// divides, for all four values (one comparison for the four and a branch that
-// is hardly ever taken).
+// subnormal results: from 1 + exp(-g) = 2^126 on (g below -87.3) it is taken of
+// 2^-32 times that (where exp overflows it is 0 and the step's NaN becomes 1, so
+// the result is -0, NaN for -inf). One comparison for the four and a branch that
+// is hardly ever taken and short: with divides behind it the epilogue's code,
+// unrolled for every tile size, cost 0.5% of a call, without the branch (the
+// scale in every value) 0.4%.
 __device__ __forceinline__ f32x4_t silu4(f32x4_t g) {
   f32x4_t d, s;
 #pragma unroll
@@ -177,7 +180,11 @@ __device__ __forceinline__ f32x4_t silu4(f32x4_t g) {
   }
   if (__builtin_expect(__any(fmaxf(fmaxf(d[0], d[1]), fmaxf(d[2], d[3])) > 0x1p126f), 0)) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) s[e] = g[e] / d[e];
+    for (int e = 0; e < 4; ++e) {
+      const float k = 0x1p-32f * d[e];
+      const float r = __builtin_amdgcn_rcpf(k);
+      if (d[e] > 0x1p126f) s[e] = g[e] * fmaf(fminf(fmaf(-k, r, 1.0f), 1.0f), r, r) * 0x1p-32f;
+    }
   }
   return s;
 }
