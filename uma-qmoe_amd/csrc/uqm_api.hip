@@ -179,14 +179,6 @@ struct MfmaPlan {
   int nb = 1, kw = 1, mw = 4, ksplit = 1;
 };
 
-// 16-route tiles per workgroup from the mean routes per expert.
-int nb_for(int enc, double mean_routes) {
-  if (mean_routes <= 16) return 1;
-  if (mean_routes <= 32) return 2;
-  if (mean_routes <= 64 || enc != UQM_BF16) return 4;
-  return 8;
-}
-
 // Enough work items (row block x route tile) for the persistent grid: 8 MMA
 // waves (128 rows per item) when there is plenty of work, 4 (64 rows), then
 // waves and workgroups along K when there is little. Every K range keeps
@@ -317,8 +309,10 @@ int grouped_tile_tokens(const uqm_expert_weights* w, int64_t T, int64_t R, int64
   const double mean = static_cast<double>(R) / static_cast<double>(active);
   // 48-route tiles when most experts would otherwise take a second, nearly
   // empty 32-route tile (every tile costs a full pass over the expert's rows)
-  // and both Q4 projections run 128-row items (the only kernels built for them);
-  // smaller tiles where the rows' scales leave no LDS for the larger ones
+  // and both Q4 projections run 128-row items (the only kernels built for them):
+  // Q4 blocks with a shared expert at 32 to 40 routes per expert, since the
+  // others and more routes take the large-tile kernel. Smaller tiles where the
+  // rows' scales leave no LDS for the larger ones.
   if (mean > 32 && mean <= 48 && w->encoding == UQM_Q4 && plan_routed(w, 3, active, T).fits) return 48;
   for (int nb = mean >= 16 ? 2 : 1; nb >= 1; --nb)
     if (plan_routed(w, nb, active, T).fits) return 16 * nb;
@@ -640,7 +634,7 @@ int run_shared(const uqm_layer_weights* layer, const uint16_t* x, int64_t T, int
     // waves (16-row items) and fill the grid; the second tile of a row block
     // runs right after the first on the same workgroup and reads the rows
     // from L2.
-    const int nb = T <= 32 ? 1 : nb_for(UQM_BF16, static_cast<double>(T));
+    const int nb = T <= 32 ? 1 : T <= 64 ? 4 : 8;
     const int ntok = 16 * nb;
     const int64_t tiles = (T + ntok - 1) / ntok;
     // Beside the routing chain, the persistent grids take 3/4 of the CUs'
@@ -753,11 +747,15 @@ static int linear_impl(int enc, const void* input, int64_t rows, const void* w, 
   a.out = output;
   a.ldo = out_features;
   // Many rows: MFMA tiles (uqm_prefill.hip), from 17 rows on for Q8, 25 for Q4
-  // and BF16. The GEMV reads the matrix again every 4 rows (18 to 25 rows cost it
-  // as much as the tiled kernel, bound by its chain of K / 128 stages, takes for
-  // up to ~300). Measured, us per call, 1408 x 2048: Q4 16 rows 12.2 vs 10.8, 24
-  // 12.1 vs 14.6, 137 12.9 vs 71; Q8 16 13.5 vs 13.8, 137 vs 100; BF16 24 16.0 vs
-  // 17.2, 137 vs 91; 768 x 2048: Q4 20 12.1 vs 10.9, 24 12.2 vs 12.6.
+  // and BF16. The GEMV reads the matrix again every 4 rows; the tiled kernel is
+  // bound by its chain of K / 128 stages up to ~300 rows. At these lines no
+  // measured matrix is slower on the tiles, of 16 to 16384 rows and K from 256 to
+  // 5632 (us per call at 25 rows, Q8 17, tiles vs GEMV): Q4 64 x 2048 12.1 vs 14.2,
+  // 1024 x 5632 26.8 vs 29.6, 4096 x 2048 12.7 vs 26.2; Q8 64 x 2048 13.2 vs 13.9,
+  // 1024 x 5632 30.8 vs 32.8, 16384 x 2048 18.6 vs 71.6; BF16 64 x 2048 13.8 vs
+  // 17.4, 4096 x 5632 38.9 vs 97.0. Large matrices gain from fewer rows on too; the
+  // narrow ones do not (1408 x 2048 Q4 16 rows 12.2 vs 10.8, 20 of 768 x 2048 12.1
+  // vs 10.9).
   // UQM_OPT_MFMA_MIN_TOKENS rules them as the expert projections (0: always GEMV).
   const int64_t min_rows = g_opt_mfma_min_tokens.load(std::memory_order_relaxed);
   if (min_rows > 0 && rows >= min_rows && rows >= (enc == UQM_Q8 ? 17 : 25) && rows <= 0x7FFFFFFF &&

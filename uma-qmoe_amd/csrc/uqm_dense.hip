@@ -15,7 +15,7 @@
 //     256 rows x 256 tokens in blocks of 128 x 64. Gate/up items take half of
 //     their rows from each matrix and give each wave the same rows of gate and
 //     of up, so the SiLU epilogue pairs them in registers;
-//   * K advances 64 elements per stage; every wave issues a quarter of each
+//   * K advances 64 elements per stage; every wave issues its share of each
 //     stage's loads (global_load_lds, 16 bytes per lane, no registers) into a
 //     ring of 4 stages of 32 KB, 3 of 48 KB or 2 of 64 KB, all but one ahead of the stage
 //     being computed;
@@ -35,12 +35,13 @@
 // token l%16, rows 4*(l/16)+i.
 #include "uqm_dense.h"
 
+#include "uqm_stage.h"
+
 #include "uqm_internal.h"
 
 namespace uqm {
 namespace {
 
-typedef __attribute__((address_space(3))) void dense_lds_t;
 
 constexpr int kStepK = 64;             // K elements per stage
 constexpr int kRowBytes = 2 * kStepK;  // one staged row
@@ -70,34 +71,18 @@ struct DenseCfg {
   static_assert((kStages - 1) * kLoadsPerWave <= 63, "outstanding loads must fit vmcnt");
 };
 
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N <= 63, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
 // Waits until at most n stages (PER loads each) of this wave's loads are
 // outstanding (loads complete in issue order; 0 <= n <= 3, wave-uniform).
 template <int PER>
 __device__ __forceinline__ void wait_stages(int n) {
   if (n >= 3)
-    wait_vm<3 * PER>();
+    wait_loads<3 * PER>();
   else if (n == 2)
-    wait_vm<2 * PER>();
+    wait_loads<2 * PER>();
   else if (n == 1)
-    wait_vm<PER>();
+    wait_loads<PER>();
   else
-    wait_vm<0>();
-}
-
-// This wave's LDS reads complete, then the workgroup barrier. (Its loads into
-// LDS are waited for separately, by stage; a plain __syncthreads would wait for
-// all of them.)
-__device__ __forceinline__ void stage_barrier() {
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), vmcnt and expcnt unlimited
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
+    wait_loads<0>();
 }
 
 // This wave's LDS reads complete. (Waited for before the next chunk's reads
@@ -107,14 +92,6 @@ __device__ __forceinline__ void stage_barrier() {
 __device__ __forceinline__ void reads_done() {
   __builtin_amdgcn_s_waitcnt(0xC07F);
   __builtin_amdgcn_sched_barrier(0);
-}
-
-// 16 bytes per lane from global memory into LDS at a wave-uniform LDS byte
-// address (lane l's bytes at lds_addr + 16 l). (A helper of its own: with the
-// builtin written in the kernel body the host compilation drops the kernels'
-// launch stubs.)
-__device__ __forceinline__ void dma16_to(const void* src, uint32_t lds_addr) {
-  __builtin_amdgcn_global_load_lds(src, reinterpret_cast<dense_lds_t*>(static_cast<uintptr_t>(lds_addr)), 16, 0, 0);
 }
 
 // Byte offset of 16-byte slot `slot` of staged row `row`.
@@ -168,11 +145,12 @@ __global__ __launch_bounds__(64 * WAVES, 2) void dense_mfma_kernel(DenseArgs a) 
     return r;
   };
 
-  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((dense_lds_t*)(lds)));
+  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((stage_lds_t*)(lds)));
 
-  // ---- loads: this wave's 4 weight and 4 activation loads of stage g ----
-  // Load d (0..15) of a region covers staged rows 8d .. 8d+7; lane l fills
-  // position l%8 of row 8d + l/8 with slot (l%8) ^ ((row >> 1) & 7). The lane's
+  // ---- loads: this wave's kLoadsA weight and kLoadsB activation loads of stage g ----
+  // Load d of a region (WAVES times the wave's loads) covers staged rows 8d ..
+  // 8d+7; lane l fills position l%8 of row 8d + l/8 with slot (l%8) ^ ((row >> 1)
+  // & 7). The lane's
   // source rows are set up once per item (clamped to the last row / token).
   // (kernel arguments read once: a scalar load in flight inside the loop would
   // make every LDS wait there a full one)
@@ -280,7 +258,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void dense_mfma_kernel(DenseArgs a) 
 
   // Stage g: chunk 1 is read while chunk 0's MFMAs run; then the wait for
   // stage g+1's loads and the barrier that hands buffer g back to the loads
-  // (stage g+4 goes there), and chunk 0 of stage g+1 is read while chunk 1's
+  // (stage g + kStages goes there), and chunk 0 of stage g+1 is read while chunk 1's
   // MFMAs run.
   const int pro = min(total, kStages);
   for (int g = 0; g < pro; ++g) issue(g);

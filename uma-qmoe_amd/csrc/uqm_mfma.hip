@@ -50,6 +50,7 @@
 #include <type_traits>
 
 #include "uqm_internal.h"
+#include "uqm_stage.h"
 
 namespace uqm {
 namespace {
@@ -190,34 +191,22 @@ __device__ __forceinline__ int a_read_off(int lane, int u) {
   }
 }
 
-// s_waitcnt with only vmcnt limited (gfx9 encoding: vmcnt bits 3:0 and 15:14).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N <= 63, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
 // Waits until at most n * PER loads are outstanding (n < NMAX, wave-uniform).
 template <int PER, int NMAX>
 __device__ __forceinline__ void wait_vmcnt_steps(int n) {
   if constexpr (NMAX > 1) {
     if (n >= NMAX - 1) {
-      wait_vmcnt<(NMAX - 1) * PER>();
+      wait_loads<(NMAX - 1) * PER>();
       return;
     }
     wait_vmcnt_steps<PER, NMAX - 1>(n);
   } else {
-    wait_vmcnt<0>();
+    wait_loads<0>();
   }
 }
 
 __device__ __forceinline__ void dma16(const void* src, void* lds_dst) {
   __builtin_amdgcn_global_load_lds(src, (lds_void_t*)(lds_dst), 16, 0, 0);
-}
-
-// Same, with the LDS destination as a (wave-uniform) LDS byte address.
-__device__ __forceinline__ void dma16_to(const void* src, uint32_t lds_addr) {
-  __builtin_amdgcn_global_load_lds(src, reinterpret_cast<lds_void_t*>(static_cast<uintptr_t>(lds_addr)), 16, 0, 0);
 }
 
 }  // namespace
@@ -705,17 +694,14 @@ hipError_t launch_nb(const MfmaArgs& a, int nb, int cus, bool dry, hipStream_t s
   if (nb <= 1) return launch_cfg<ENC, NMAT, MW, 1, KW>(a, cus, dry, stream);
   if constexpr (KW == 1) {
     if (nb <= 2) return launch_cfg<ENC, NMAT, MW, 2, KW>(a, cus, dry, stream);
-    if constexpr (MW == 8) {
-      // 48-route tiles; the kernel's tile size must equal the tile list's
+    if constexpr (ENC == kQ4 && MW == 8) {
+      // 48-route tiles (Q4); the kernel's tile size must equal the tile list's
       if (nb == 3) return launch_cfg<ENC, NMAT, MW, 3, KW>(a, cus, dry, stream);
     }
-    if constexpr (MW == 4) {
-      if (nb == 3) return hipErrorInvalidValue;
-      if (nb <= 4) return launch_cfg<ENC, NMAT, MW, 4, KW>(a, cus, dry, stream);
-      // 128-route tiles exist for BF16 only (a smaller kernel tile would drop routes)
-      if constexpr (ENC == kBF16) {
-        if (nb <= 8) return launch_cfg<ENC, NMAT, MW, 8, KW>(a, cus, dry, stream);
-      }
+    // 64- and 128-token tiles: the BF16 shared expert
+    if constexpr (ENC == kBF16 && MW == 4) {
+      if (nb == 4) return launch_cfg<ENC, NMAT, MW, 4, KW>(a, cus, dry, stream);
+      if (nb == 8) return launch_cfg<ENC, NMAT, MW, 8, KW>(a, cus, dry, stream);
     }
   }
   return hipErrorInvalidValue;

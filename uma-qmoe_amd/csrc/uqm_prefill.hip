@@ -20,14 +20,14 @@
 //     converted while this one's MFMAs run, each tile's B operands are read
 //     during the tile before, its sums folded during the one after);
 //   * activations come through LDS (global_load_lds, 16 bytes per lane, one
-//     128-element group of all routes per stage) in a ring of 2 to 4 stages,
+//     128-element group of all routes per stage) in a ring of 2 to 6 stages,
 //     and the group's scales with them, so that a lane reads the scales of its
 //     4 rows as one vector;
 //   * an expert's routes are split evenly (route_tile_step), and the loop is
 //     compiled for every tile size from 1 to 9 sixteens, so that padding stays
 //     below 16 routes per tile;
-//   * one work item per workgroup and two workgroups per CU (72 KB of ring, at
-//     most 256 VGPRs): the hardware dispatcher balances items of different
+//   * one work item per workgroup and two workgroups per CU (at most 78 KB of
+//     ring and 256 VGPRs): the hardware dispatcher balances items of different
 //     sizes, and one workgroup's start and end run under the other's MFMAs.
 // What bounds it (OLMoE shapes, 4095 tokens): without its loads the loop runs
 // at ~1.5 PFLOP/s, the rate of a large library product on this card; the
@@ -50,20 +50,21 @@
 // of a lane's 16-byte weight loads, the same for A and B.
 #include "uqm_prefill.h"
 
+#include "uqm_stage.h"
+
 #include <type_traits>
 
 namespace uqm {
 namespace {
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void prefill_lds_t;
 
 constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kRowBytes = 256;                  // one staged activation row: 128 bf16
 constexpr int kTileBytes = 16 * kRowBytes;      // 16 routes of one stage
 constexpr int kMaxTT = kPrefillTileTokens / 16;  // 16-route tiles per item
-constexpr int kRingTiles = 18;                  // 72 KB
+constexpr int kRingTiles = 18;                  // 72 KB of activations
 constexpr int kMaxStages = 6;
 
 // Stages of the ring for items of TT tiles: small items run through a stage
@@ -189,31 +190,6 @@ __device__ __forceinline__ f32x4_t silu4(f32x4_t g) {
   return s;
 }
 
-// s_waitcnt with only vmcnt limited (gfx9 encoding: vmcnt bits 3:0 and 15:14).
-template <int N>
-__device__ __forceinline__ void wait_loads() {
-  static_assert(N >= 0 && N <= 63, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-// This wave's LDS reads complete, then the workgroup barrier (loads into LDS
-// are waited for separately, by stage).
-__device__ __forceinline__ void stage_barrier() {
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), vmcnt and expcnt unlimited
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-// 16 or 4 bytes per lane from global memory into LDS at a wave-uniform LDS
-// byte address (lane l's bytes at lds_addr + 16 l or + 4 l).
-__device__ __forceinline__ void dma16(const void* src, uint32_t lds_addr) {
-  __builtin_amdgcn_global_load_lds(src, reinterpret_cast<prefill_lds_t*>(static_cast<uintptr_t>(lds_addr)), 16, 0, 0);
-}
-__device__ __forceinline__ void dma4(const void* src, uint32_t lds_addr) {
-  __builtin_amdgcn_global_load_lds(src, reinterpret_cast<prefill_lds_t*>(static_cast<uintptr_t>(lds_addr)), 4, 0, 0);
-}
-
 // One work item of TT 16-route tiles: rows of row block rb of `expert`, the
 // nt <= 16 TT routes listed in LDS.
 template <int ENC, int NMAT, int MODE, int TT>
@@ -231,7 +207,7 @@ __device__ __forceinline__ void run_item(const MfmaArgs& a, unsigned char* lds, 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int q = lane >> 4, t16 = lane & 15;
-  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((prefill_lds_t*)(lds)));
+  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((stage_lds_t*)(lds)));
   const int S = static_cast<int>(a.K / 128);
   const int rows = static_cast<int>(a.rows);
   const uint32_t row_bytes = static_cast<uint32_t>(S) * E::kGroupBytes;
@@ -279,10 +255,10 @@ __device__ __forceinline__ void run_item(const MfmaArgs& a, unsigned char* lds, 
     for (int j = 0; j < TT; ++j) {
       uint32_t o = xoff[j];
       asm("" : "+v"(o));  // (extended to 64 bits by the load itself, not kept extended)
-      dma16(xg + o, buf + (16 * j + 4 * wave) * kRowBytes);
+      dma16_to(xg + o, buf + (16 * j + 4 * wave) * kRowBytes);
     }
     if constexpr (kScaled)
-      dma4(ssrc + g / gdiv, __builtin_amdgcn_readfirstlane(buf + TT * kTileBytes + wave * 256));
+      dma4_to(ssrc + g / gdiv, __builtin_amdgcn_readfirstlane(buf + TT * kTileBytes + wave * 256));
   };
   auto load_weights = [&](int g, uint4 (&v)[2][L]) {
 #pragma unroll
