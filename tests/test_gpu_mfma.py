@@ -9,6 +9,7 @@ bf16 outputs agree to a few bf16 ulps.
 
 from __future__ import annotations
 
+import ctypes
 import sys
 from dataclasses import replace
 
@@ -95,6 +96,22 @@ def routes(t, k, e, seed, hot=None, hot_share=0.0):
     return idx, w
 
 
+def plan_of(layer, tokens, top_k, shared=0):
+    """The kernels a call takes under the current options (uqm_moe_layer_plan):
+    a test that means one of them says so."""
+    weights = _native.LayerWeights(layer.descriptor(), 16, top_k, 0, int(shared > 0), shared, 16, 16, 16, 16)
+    out = _native.LayerPlan()
+    _native.check(_native.library().uqm_moe_layer_plan(ctypes.byref(weights), tokens, ctypes.byref(out)), "plan")
+    return out
+
+
+def dense_plan(layer, tokens, top_k, shared):
+    p = plan_of(layer, tokens, top_k, shared)
+    return (p.gate_up_rows, p.gate_up_tokens), (p.down_rows, p.down_tokens, p.down_split)
+
+
+LARGE = 144  # routed_tile of the large-tile kernel
+
 STREAM_DEFAULT = 32  # UQM_OPT_STREAM_MAX_ROUTES default (routes per call)
 STREAM_ALWAYS = 1 << 30
 
@@ -142,13 +159,16 @@ def streamed(ext, fn, threshold=STREAM_ALWAYS):
 @pytest.mark.parametrize("encoding", ["q4_group128", "q8_group128", "bf16_le"])
 @pytest.mark.parametrize("t", [2, 16, 37, 100, 300])
 def test_routed_matches_oracle_and_gemv(mfma_on, encoding, t):
-    """Routed experts on the grouped-GEMM kernel against the oracle and the
-    GEMV path."""
+    """Routed experts on the grouped-GEMM kernels against the oracle and the
+    GEMV path: 16-route tiles, 32-route tiles (Q8 and BF16 at 25 routes per
+    expert), the large tiles."""
     ext = mfma_on
     shape = replace(MID, encoding=encoding)
     note(f"mfma routed {encoding} t={t}")
     layer = syn.build_experts(shape, seed=t)
     dl = to_dev(layer)
+    tile = {2: 16, 16: 16, 37: 16, 100: LARGE if encoding == "q4_group128" else 32, 300: LARGE}[t]
+    assert plan_of(dl, t, shape.top_k).routed_tile == tile
     x = syn.hidden_states(shape, t, seed=t)
     idx, w = routes(t, shape.top_k, shape.num_experts, 100 + t)
     got, gemv = both_paths(ext, lambda: ext.moe_forward(dl, x.to(DEV), idx.to(DEV), w.to(DEV)))
@@ -234,12 +254,22 @@ def test_qwen_block_stream_decode(mfma_on, t):
 def test_hot_expert_spans_many_tiles(mfma_on, encoding):
     """One expert takes ~85% of 300 tokens (k=2): it is split into many route
     tiles that share its weight rows; idle experts get no tile."""
-    ext = mfma_on
+    hot_expert(mfma_on, encoding, 300, LARGE)
+
+
+@pytest.mark.parametrize("encoding,t", [("q4_group128", 180), ("q8_group128", 280), ("bf16_le", 250)])
+def test_hot_expert_spans_32_route_tiles(mfma_on, encoding, t):
+    """The same below the large tiles' range: the hot expert takes five to
+    eight tiles of 32 routes."""
+    hot_expert(mfma_on, encoding, t, 32)
+
+
+def hot_expert(ext, encoding, t, tile):
     shape = replace(MID, encoding=encoding, top_k=2)
-    note(f"mfma hot expert {encoding}")
+    note(f"mfma hot expert {encoding} t={t}")
     layer = syn.build_experts(shape, seed=5)
     dl = to_dev(layer)
-    t = 300
+    assert plan_of(dl, t, 2).routed_tile == tile
     x = syn.hidden_states(shape, t, seed=5)
     idx, w = routes(t, 2, shape.num_experts, 7, hot=5, hot_share=0.85)
     got = ext.moe_forward(dl, x.to(DEV), idx.to(DEV), w.to(DEV))
@@ -258,16 +288,17 @@ def test_hot_expert_spans_many_tiles(mfma_on, encoding):
 
 def test_48_route_tiles(mfma_on):
     """Q4, 32 experts x 1024 rows, 300 tokens top-4: 37.5 routes per expert on
-    average, so the routed projections take 48-route tiles (3 x 16 tokens per
-    MFMA item; every expert's rows x 32 experts fill the 256 CUs). One expert
-    takes ~30% of the tokens (three tiles, the last one partial); the others
-    fill 25-46 of one tile. Against the oracle and the GEMV path."""
+    average (without a shared expert beside them the large tiles; the 48-route
+    tiles of the same routes are in the block test below). One expert takes
+    ~30% of the tokens; the others 25-46. Against the oracle and the GEMV
+    path."""
     ext = mfma_on
     shape = syn.MoEShape("tile48", 2048, 32, 4, 1024)
     note("mfma 48-route tiles")
     layer = syn.build_experts(shape, seed=11)
     dl = to_dev(layer)
     t = 300
+    assert plan_of(dl, t, 4).routed_tile == LARGE
     x = syn.hidden_states(shape, t, seed=11)
     idx, w = routes(t, 4, shape.num_experts, 13, hot=3, hot_share=0.3)
     counts = torch.bincount(idx.flatten(), minlength=shape.num_experts)
@@ -276,6 +307,37 @@ def test_48_route_tiles(mfma_on):
     ref = om.streaming_reference(x, idx, w, 0, syn.DeviceLayerReader({0: layer}), num_experts=shape.num_experts)
     close(got, ref, "48-route tiles")
     close(got, got_g, "48-route tiles mfma vs gemv", rel=5e-3, mx=1e-2)
+
+
+@pytest.mark.parametrize("hidden,e,inter,t", [(2048, 32, 1024, 300), (1152, 40, 896, 380)])
+def test_48_route_tiles_of_a_block(mfma_on, hidden, e, inter, t):
+    """Q4 blocks with a shared expert at 37.5 and 38 routes per expert: 48-route
+    tiles (3 x 16 tokens per MFMA item; every expert's rows x the experts fill
+    the 256 CUs), with even and odd numbers of scale groups in both projections.
+    About 30% of the tokens (those with a large first element) send a route to
+    one expert: three tiles, the last one partial. Against the oracle on
+    sampled tokens and the GEMV path on all."""
+    ext = mfma_on
+    shape = syn.MoEShape("tile48_block", hidden, e, 4, inter, 768)
+    note(f"mfma 48-route tiles of a block {hidden}")
+    layer = syn.build_experts(shape, device=DEV)
+    dense = syn.build_dense(shape, device=DEV)
+    dense.router[:, 0] = 0
+    dense.router[3, 0] = 2
+    assert plan_of(layer, t, 4, 768).routed_tile == 48
+    x = syn.hidden_states(shape, t, seed=11)
+    x[:, 0] = 0
+    x[torch.rand(t, generator=torch.Generator().manual_seed(1)) < 0.3, 0] = 4
+    (out, logits, weights, indices), (out_g, *_rest) = both_paths(
+        ext, lambda: ext.moe_layer(layer, dense, x.to(DEV), shape.top_k))
+    counts = torch.bincount(indices.flatten().cpu(), minlength=e)
+    assert counts.argmax() == 3 and counts.max() > 96 and counts.min() > 0
+    assert_weights_follow_logits(logits, weights, indices, False, "48-route block")
+    close(out, out_g, "48-route block mfma vs gemv", rel=5e-3, mx=1e-2)
+    pick = torch.arange(0, t, 23)
+    ref, *_ = om.qwen_block(x[pick], layout_of(shape, dense_cpu(dense)), syn.DeviceLayerReader({0: layer}), 0,
+                            routes=(weights.cpu()[pick], indices.cpu()[pick]))
+    close(out.cpu()[pick], ref, "48-route block sampled tokens vs oracle")
 
 
 def random_experts(encoding, e, hidden, inter, seed):
@@ -323,12 +385,14 @@ def test_q4_odd_group_count(mfma_on, t):
     256; the MID shape's gate/up and the c2 block's at batch 16 and 32 take
     them) and run one group per step. The planner takes (gate/up; down): t=6
     64-row items (down with two K-split partials when the items are few); t=32
-    128-row items, 16-route tiles; t=200 32-route tiles; t=400 48-route tiles.
-    Against the oracle and the GEMV path."""
+    128-row items, 16-route tiles; t=200 32-route tiles; t=400 the large tiles
+    (48-route tiles: the block test above). Against the oracle and the GEMV
+    path."""
     ext = mfma_on
     note(f"mfma odd group count t={t}")
     layer = syn.build_experts(ODD, seed=60 + t)
     dl = to_dev(layer)
+    assert plan_of(dl, t, ODD.top_k).routed_tile == {6: 16, 32: 16, 200: 32, 400: LARGE}[t]
     x = syn.hidden_states(ODD, t, seed=60 + t)
     idx, w = routes(t, ODD.top_k, ODD.num_experts, 160 + t)
     got, gemv = both_paths(ext, lambda: ext.moe_forward(dl, x.to(DEV), idx.to(DEV), w.to(DEV)))
@@ -407,8 +471,8 @@ def test_dense_shared_expert(mfma_on, which, t):
     half full) and 1344 shared rows (21 K stages in the down projection: no K
     split); c2 at 200 tokens splits the down projection's K in four; at 384
     tokens the gate/up takes 8-wave items (the second 256-token tile half
-    full); at 1000 tokens both projections take 8-wave items, the down
-    projection with its K split in four. Against the oracle on sampled tokens
+    full); at 1000 tokens both projections take 8-wave items, the gate/up of
+    256 rows, the down projection with its K split in two. Against the oracle on sampled tokens
     (the last token always among them) and against the GEMV path on every
     token."""
     ext = mfma_on
@@ -416,6 +480,9 @@ def test_dense_shared_expert(mfma_on, which, t):
     note(f"dense shared expert {which} t={t}")
     layer = syn.build_experts(shape, device=DEV)
     dense = syn.build_dense(shape, device=DEV)
+    small = ((128, 128), (128, 128, 1 if which == "ragged" else 4))
+    assert dense_plan(layer, t, shape.top_k, shape.shared_intermediate) == {
+        384: ((128, 256), (128, 128, 4)), 1000: ((256, 256), (128, 256, 2))}.get(t, small)
     x = syn.hidden_states(shape, t, seed=90 + t)
     (out, logits, weights, indices), (out_g, *_rest) = both_paths(
         ext, lambda: ext.moe_layer(layer, dense, x.to(DEV), shape.top_k))
@@ -437,6 +504,8 @@ def test_c4_prefill_512_tokens(mfma_on):
     note("mfma c4 T=512")
     layer = syn.build_experts(shape, device=DEV)
     dense = syn.build_dense(shape, device=DEV)
+    assert plan_of(layer, 512, shape.top_k, shape.shared_intermediate).routed_tile == 48
+    assert dense_plan(layer, 512, shape.top_k, shape.shared_intermediate) == ((128, 256), (128, 256, 4))
     x = syn.hidden_states(shape, 512, seed=4)
     (out, logits, weights, indices), (out_g, *_rest) = both_paths(
         ext, lambda: ext.moe_layer(layer, dense, x.to(DEV), shape.top_k))

@@ -15,7 +15,8 @@ import torch
 from oracle import codec as oc
 from oracle import moe as om
 from test_gpu_kernels import assert_bf16_rounded
-from test_gpu_mfma import DEV, RAGGED, close, dense_cpu, layout_of, mfma_on, note, to_dev  # noqa: F401
+from test_gpu_mfma import (DEV, LARGE, RAGGED, close, dense_cpu, dense_plan, layout_of, mfma_on, note,  # noqa: F401
+                           plan_of, to_dev)
 from uma_qmoe_amd import _native
 from uma_qmoe_amd import synthetic as syn
 
@@ -44,6 +45,7 @@ def test_tile_sizes_against_oracle(mfma_on, encoding, hidden, inter):  # noqa: F
     layer = syn.build_experts(shape, seed=hidden)
     idx, w = skewed_routes(COUNTS, inter)
     assert idx.numel() / len(COUNTS) >= 44  # the large-tile kernel's range for every encoding
+    assert plan_of(layer, idx.shape[0], 1).routed_tile == LARGE
     x = syn.hidden_states(shape, idx.shape[0], seed=3)
     got = mfma_on.moe_forward(to_dev(layer), x.to(DEV), idx.to(DEV), w.to(DEV))
     ref = om.streaming_reference(x, idx, w, 0, syn.DeviceLayerReader({0: layer}), num_experts=len(COUNTS))
@@ -61,6 +63,7 @@ def test_wide_scale_groups_and_dropped_routes(mfma_on, encoding):  # noqa: F811
     idx = torch.stack([torch.randperm(5, generator=g)[:2] for _ in range(333)])
     w = torch.rand(333, 2, generator=g).to(torch.bfloat16)
     x = syn.hidden_states(shape, 333, seed=5)
+    assert plan_of(layer, 333, 2).routed_tile == LARGE
     dropped = idx.clone()
     dropped[::5, 1] = -1
     dropped[1::7, 0] = 5
@@ -81,6 +84,7 @@ def test_infinities_and_nan_stay_in_their_token(mfma_on):  # noqa: F811
     idx = (torch.arange(t) % 2).view(-1, 1)
     w = torch.ones(t, 1, dtype=torch.bfloat16)
     x = syn.hidden_states(shape, t, seed=6)
+    assert plan_of(layer, t, 1).routed_tile == LARGE
     clean = mfma_on.moe_forward(layer, x.to(DEV), idx.to(DEV), w.to(DEV)).cpu()
     bad = x.clone()
     bad[0, 3] = float("nan")  # token 0 pads expert 0's last tile
@@ -114,6 +118,7 @@ def test_silu_of_large_negative_gates(mfma_on):  # noqa: F811
     layer = replace(syn.build_experts(shape), gate=gate.to(torch.bfloat16), up=up.to(torch.bfloat16),
                     down=down.to(torch.bfloat16))
     idx = (torch.arange(t) // 8 % 2).view(-1, 1)
+    assert plan_of(layer, t, 1).routed_tile == LARGE
     got = mfma_on.moe_forward(to_dev(layer), x.to(DEV), idx.to(DEV), torch.ones(t, 1, dtype=torch.bfloat16, device=DEV))
     g = gates.double()
     ref = g / (1 + torch.exp(-g)) * 2.0 ** 100
@@ -131,6 +136,7 @@ def test_block_replays_from_a_graph(mfma_on):  # noqa: F811
     layer = syn.build_experts(shape, device=DEV)
     dense = syn.build_dense(shape, device=DEV)
     x = syn.hidden_states(shape, 900, device=DEV)  # 3600 routes, 450 per expert
+    assert plan_of(layer, 900, shape.top_k, shape.shared_intermediate).routed_tile == LARGE
     ws = ext.new_workspace(DEV, 900, shape.hidden, shape.intermediate, shape.shared_intermediate, 8, shape.top_k)
     ref = ext.moe_layer(layer, dense, x, shape.top_k, workspace=ws)[0].clone()
     torch.cuda.synchronize()
@@ -145,11 +151,12 @@ def test_block_replays_from_a_graph(mfma_on):  # noqa: F811
         ext.moe_layer(layer, dense, x, shape.top_k, workspace=ws)
 
 
-# rows: the first that takes the tiles, both sides of one 16-row tile, of the
-# largest tile, several tiles; out features: not a multiple of the 128-row block
-# (16, 1424), below it (64), and one the tiles do not take (1420)
+# rows: both sides of the first that takes the tiles (Q8 17, the others 25), of
+# one 16-row tile, of the largest tile, several tiles; out features: not a
+# multiple of the 128-row block (16, 1424), below it (64), and one the tiles do
+# not take (1420)
 @pytest.mark.parametrize("encoding", ["q4_group128", "q8_group128", "bf16_le"])
-@pytest.mark.parametrize("rows,n,k", [(25, 1424, 256), (33, 16, 640), (144, 64, 2048), (145, 1424, 384),
+@pytest.mark.parametrize("rows,n,k", [(16, 64, 256), (17, 1424, 256), (24, 64, 2048), (25, 1424, 256), (33, 16, 640), (144, 64, 2048), (145, 1424, 384),
                                       (700, 1420, 256), (1000, 1424, 512)])
 def test_linear_many_rows(hip_ext, encoding, rows, n, k):
     note(f"linear {encoding} rows={rows} n={n} k={k}")
@@ -168,6 +175,42 @@ def test_linear_many_rows(hip_ext, encoding, rows, n, k):
         deq = data[0].float().numpy()
         got = hip_ext.bf16_linear(xd, wd)
     assert_bf16_rounded(got, x.float() @ torch.from_numpy(deq).T, "linear")
+
+
+@pytest.mark.parametrize("encoding", ["q4_group128", "q8_group128"])
+def test_lowest_codes_on_the_tiles(hip_ext, encoding):
+    """The codecs never write the lowest code (-8, -128); the tiles' conversions
+    take it as two's complement all the same."""
+    note(f"lowest codes {encoding}")
+    rows, n, k = 40, 64, 256
+    g = torch.Generator().manual_seed(12)
+    low = -8 if encoding == "q4_group128" else -128
+    codes = torch.randint(low, -low, (n, k), generator=g, dtype=torch.int8)
+    codes[:, ::5] = low
+    scales = torch.rand(n * k // 128, generator=g) * 1e-2
+    x = torch.randn(rows, k, generator=g).to(torch.bfloat16)
+    data = (codes[:, 0::2] & 15 | codes[:, 1::2] << 4).view(torch.uint8) if low == -8 else codes
+    linear = hip_ext.q4_linear if low == -8 else hip_ext.q8_linear
+    got = linear(x.to(DEV), data.contiguous().to(DEV), scales.to(DEV), n, k, 128)
+    deq = codes.float() * scales.repeat_interleave(128).view(n, k)
+    assert_bf16_rounded(got, x.float() @ deq.T, "lowest codes")
+
+
+def test_linear_to_an_unaligned_output(hip_ext):
+    """An output that is not 8-byte aligned stays on the GEMV: bit for bit its
+    rows in calls of four."""
+    note("linear unaligned output")
+    rows, n, k = 136, 64, 512
+    g = torch.Generator().manual_seed(13)
+    data, scales = syn.encode_projection(torch.randn(1, n, k, generator=g) * 0.02, "q4_group128")
+    w, s = data[0].to(DEV), scales[0].to(DEV)
+    x = torch.randn(rows, k, generator=g).to(torch.bfloat16).to(DEV)
+    gemv = torch.cat([hip_ext.q4_linear(x[i:i + 4], w, s, n, k, 128) for i in range(0, rows, 4)])
+    buf = torch.zeros(rows * n + 2, dtype=torch.bfloat16, device=DEV)
+    _native.check(hip_ext.lib.uqm_q4_linear(x.data_ptr(), rows, w.data_ptr(), s.data_ptr(), n, k, 128,
+                                            buf.data_ptr() + 2, torch.cuda.current_stream().cuda_stream), "linear")
+    assert torch.equal(buf[1:-1].view(rows, n), gemv)
+    assert buf[0] == 0 and buf[-1] == 0
 
 
 @pytest.mark.parametrize("encoding", ["q4_group128", "q8_group128", "bf16_le"])
@@ -202,11 +245,13 @@ def test_dense_256_row_items(mfma_on, which, t):  # noqa: F811
     ragged shape's gate/up at 4300 tokens (1344 rows: the last 128-row half
     block half full; 17 token tiles, the last one partial) and for its down
     projection at 9700 (1088 rows: 64 in the last block), and for both c2
-    projections at 2100 tokens (K split in four)."""
+    projections at 2100 tokens (K split in two)."""
     shape = RAGGED if which == "ragged" else syn.C2
     note(f"dense 256 rows {which} t={t}")
     layer = syn.build_experts(shape, device=DEV)
     dense = syn.build_dense(shape, device=DEV)
+    down = {4300: (128, 256, 1), 9700: (256, 256, 1), 2100: (256, 256, 2)}[t]
+    assert dense_plan(layer, t, shape.top_k, shape.shared_intermediate) == ((256, 256), down)
     x = syn.hidden_states(shape, t, seed=t)
     out, _logits, weights, indices = mfma_on.moe_layer(layer, dense, x.to(DEV), shape.top_k)
     pick = torch.randperm(t, generator=torch.Generator().manual_seed(t))[:24]
