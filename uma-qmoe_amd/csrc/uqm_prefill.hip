@@ -152,8 +152,9 @@ __device__ __forceinline__ int x_slot(int q, int S) {
 // the next one (or the other way round), so their positions are distinct when
 // {swizzle(rows 0-3, 12-15)} and {swizzle(rows 4-11) ^ (slot step from one
 // quadrant to the next)} are: with the row itself for steps of 1 and 2 (BF16,
-// Q8), with bit 2 of the row taken from bit 3 for steps of 4 (Q4). (No bank
-// conflicts in the counters.) An aligned group of four positions holds an
+// Q8), with bit 2 of the row taken from bit 3 for steps of 4 (Q4). (The bank
+// conflicts in the counters are the weights' reorder, 2 cycles per ds_bpermute.)
+// An aligned group of four positions holds an
 // aligned group of four slots, so that the four neighbouring lanes which the
 // address unit takes together load 64 contiguous bytes: 16 cache accesses per
 // load of 64 lanes, against 64 when the slots of a group are stored apart.
